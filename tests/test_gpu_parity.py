@@ -64,6 +64,72 @@ def test_exact_mode_is_bit_identical_to_the_fused_reference(tk, orc, p):
         tk.set_mode(tk.FAST)
 
 
+# Row blocks per workgroup 1 to 4 (375, 750 and 1000 rows by 1024 outputs take 2, 3 and 4), ragged rows,
+# outputs and inputs (64 inputs per stage; one more, one less, several stages of the ring and a bit).
+EXACT_TILES = [(1, 64, 16), (17, 65, 40), (33, 63, 33), (93, 448, 70), (375, 193, 1021), (750, 257, 1024),
+               (745, 96, 1010), (1000, 128, 1024), (990, 321, 1020)]
+
+
+@pytest.mark.parametrize("m,k,n", EXACT_TILES)
+@pytest.mark.parametrize("p", [F32, F16, BF16, INT8, Q8_0])
+def test_exact_products_on_each_tile_are_the_fused_reference(tk, orc, p, m, k, n):
+    """Every tile of the exact kernel, rows that are 16 bytes aligned and rows that are not: the fused
+    reference's bits."""
+    import torch
+
+    import telmo_amd
+
+    if p == Q8_0:
+        k = -(-k // 32) * 32
+    a, c0, bias = orc.random(m * k, 1), orc.random(m * n, 4), orc.random(n, 3)
+    values, scales = orc.encode(orc.random(n * k, 2), n, k, p)
+    want = c0.copy()
+    assert orc.matmul(True, a, k, m, values, scales, p, n, k, want, n, bias, SILU, 0.5, True) == 0
+    w = telmo_amd.PackedWeights.from_parts(tk, n, k, telmo_amd.Precision(p), values, scales)
+    tk.set_mode(tk.EXACT)
+    try:
+        for lda, off in ((k, 0), (-(-k // 4) * 4, 0), (k + 3, 1)):
+            say("exact tile", p, m, k, n, lda, off)
+            rows = np.zeros((m, lda), np.float32)
+            rows[:, :k] = a.reshape(m, k)
+            ad = torch.from_numpy(np.concatenate([np.zeros(off, np.float32), rows.reshape(-1)])).cuda()[off:]
+            cd = torch.from_numpy(c0.copy()).cuda()
+            tk.matmul_device(ad, lda, m, w, cd, n,
+                             telmo_amd.Epilogue(bias=torch.from_numpy(bias).cuda(), act=telmo_amd.Act.SILU, scale=0.5,
+                                                accumulate=True))
+            tk.synchronize()
+            assert np.array_equal(cd.cpu().numpy().view(np.uint32), want.view(np.uint32)), (p, m, k, n, lda, off)
+    finally:
+        tk.set_mode(tk.FAST)
+        w.close()
+
+
+@pytest.mark.parametrize("k", [31, 64, 65, 200])
+def test_exact_sums_keep_subnormals_signed_zeros_and_infinities(tk, orc, k):
+    """Sums that underflow to -0, subnormal inputs and products, infinities and NaN: the fused
+    reference's bits (any NaN for a NaN), whatever the padding of the last stage."""
+    import telmo_amd
+
+    rng = np.random.default_rng(k)
+    m, n = 20, 40
+    a = np.ldexp(rng.uniform(-1, 1, (m, k)), rng.integers(-149, 20, (m, k))).astype(np.float32)
+    a[0], a[1], a[2] = -1e-30, 0.0, -0.0
+    a[3, k // 2], a[4, k - 1], a[5, 0] = np.inf, -np.inf, np.nan
+    b = np.ldexp(rng.uniform(-1, 1, (n, k)), rng.integers(-149, 20, (n, k))).astype(np.float32)
+    b[0] = 1e-30  # row 0 by output 0: each product is below the least subnormal, the sum -0
+    values, _ = orc.encode(b.reshape(-1), n, k, F32)
+    want = np.zeros(m * n, np.float32)
+    assert orc.matmul(True, a.reshape(-1), k, m, values, None, F32, n, k, want, n, None, NONE, 1.0, False) == 0
+    assert want.view(np.uint32)[0] == 0x80000000
+    w = telmo_amd.PackedWeights.from_parts(tk, n, k, telmo_amd.Precision.F32, values, None)
+    got = np.zeros(m * n, np.float32)
+    tk.linear(a.reshape(-1), m, w, got)
+    w.close()
+    nan = np.isnan(want)
+    assert np.array_equal(np.isnan(got), nan)
+    assert np.array_equal(got.view(np.uint32)[~nan], want.view(np.uint32)[~nan])
+
+
 # (700, 2048, 1000) and (1300, 2048, 700) take the k-split kernel with 48- and 64-row tiles;
 # (100, 1000, 4100) the direct kernel on a wide product with fewer 64 x 64 tiles than CUs.
 FAST_SHAPES = [(1, 1, 1), (3, 7, 5), (8, 64, 16), (9, 64, 16), (13, 100, 50), (64, 128, 96), (130, 1000, 255),
