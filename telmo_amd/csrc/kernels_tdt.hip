@@ -664,6 +664,33 @@ __device__ __forceinline__ bool wait_words(const uint64_t *const (&p)[N], uint32
     }
 }
 
+// Where the 16 hi digits of inputs 64 t + 16 g .. of row r sit in the 16-row digit layout (the lo digits
+// 1024 bytes on): k-block t's 2 KB, then 256 bytes per group g with the rows' 16 bytes permuted by (t, g),
+// so that the lanes of a wavefront writing one row's chunks (16 pairs of t and g) meet 16 bank groups
+// instead of one; the 16 rows that an MFMA operand read takes are all there either way.
+__device__ __forceinline__ int digit_slot(int t, int g, int r) {
+    return t * 2048 + g * 256 + ((r ^ (((t & 3) << 2) | g)) << 4);
+}
+// The four digits of chunk c (inputs 4 c ..) of row r.
+__device__ __forceinline__ int digit_chunk(int c, int r) { return digit_slot(c >> 4, (c >> 2) & 3, r) + (c & 3) * 4; }
+
+// wait_words for the words at base + off[i].
+template <int N>
+__device__ __forceinline__ bool wait_offsets(const uint64_t *base, const uint32_t (&off)[N], uint32_t need,
+                                             const uint32_t (&tag)[N], uint64_t (&w)[N], const int32_t *err,
+                                             uint64_t deadline) {
+    for (int round = 0; need; round++) {
+#pragma unroll
+        for (int i = 0; i < N; i++)
+            if (need >> i & 1) w[i] = word_load(base + off[i]);
+#pragma unroll
+        for (int i = 0; i < N; i++)
+            if ((need >> i & 1) && (uint32_t)(w[i] >> 32) == tag[i]) need &= ~(1u << i);
+        if (need && (round & 15) == 15 && ((uint64_t)wall_clock64() > deadline || load_i(err) != 0)) return false;
+    }
+    return true;
+}
+
 // Copies np panels from p0 on of a matrix into LDS, panel pi's k-block t at (pi KB + t) * 1024.
 __device__ __forceinline__ void copy_panels(uint8_t *dst, const ResMat &m, int p0, int np) {
     const int per = m.KB * 64, total = np * per;
@@ -979,7 +1006,7 @@ __global__ __launch_bounds__(RES_THREADS) void tdt_resident_kernel(ResArgs a) {
                         if (c < KBJ4 * 16) {  // zero digits past the row (z is 0 there)
                             uint32_t hi, lo;
                             digits4(z[i].x, z[i].y, z[i].z, z[i].w, ex, hi, lo);
-                            uint8_t *d = sq + (c >> 4) * 2048 + ((c & 15) >> 2) * 256 + r * 16 + (c & 3) * 4;
+                            uint8_t *d = sq + digit_chunk(c, r);
                             *reinterpret_cast<uint32_t *>(d) = hi;
                             *reinterpret_cast<uint32_t *>(d + 1024) = lo;
                         }
@@ -1011,9 +1038,9 @@ __global__ __launch_bounds__(RES_THREADS) void tdt_resident_kernel(ResArgs a) {
                         gemv::v4i H[2], L[2];
 #pragma unroll
                         for (int hh = 0; hh < 2; hh++) {
-                            const int off = off0 + hh * 512;
-                            const long ah = *reinterpret_cast<const long *>(sq + t * 2048 + off);
-                            const long al = *reinterpret_cast<const long *>(sq + t * 2048 + 1024 + off);
+                            const int off = off0 + hh * 512, dig = digit_slot(t, 2 * hh + (g >> 1), j16) + 8 * (g & 1);
+                            const long ah = *reinterpret_cast<const long *>(sq + dig);
+                            const long al = *reinterpret_cast<const long *>(sq + 1024 + dig);
                             const long wv = *reinterpret_cast<const long *>(wb + (size_t)t * 1024 + off);
                             H[hh] = __builtin_amdgcn_mfma_i32_16x16x32_i8(ah, wv, gemv::v4i{0, 0, 0, 0}, 0, 0, 0);
                             L[hh] = __builtin_amdgcn_mfma_i32_16x16x32_i8(al, wv, gemv::v4i{0, 0, 0, 0}, 0, 0, 0);
@@ -1036,8 +1063,8 @@ __global__ __launch_bounds__(RES_THREADS) void tdt_resident_kernel(ResArgs a) {
                         gemv::v4i ah[4], al[4], wv[4];
 #pragma unroll
                         for (int u = 0; u < 4; u++) {
-                            ah[u] = *reinterpret_cast<const gemv::v4i *>(sq + (t0 + u) * 2048 + lane * 16);
-                            al[u] = *reinterpret_cast<const gemv::v4i *>(sq + (t0 + u) * 2048 + 1024 + lane * 16);
+                            ah[u] = *reinterpret_cast<const gemv::v4i *>(sq + digit_slot(t0 + u, lane >> 4, j16));
+                            al[u] = *reinterpret_cast<const gemv::v4i *>(sq + 1024 + digit_slot(t0 + u, lane >> 4, j16));
                             wv[u] = *reinterpret_cast<const gemv::v4i *>(wb + (size_t)min(t0 + u, KBJ - 1) * 1024);
                         }
 #pragma unroll
@@ -1416,7 +1443,8 @@ struct MultiShared {
     int st[MS_MAX][5];
     uint32_t n[MS_MAX], pin_n[MS_MAX];
     int dec[MS_MAX][RES_DEC];
-    int emit[MS_MAX], nemit;
+    int nemit;
+    __attribute__((aligned(16))) gemv::v4i part[RES_WAVES - 1][2][4 * MS_MAX];  // rows_sums' partial sums
     int abort;
 };
 
@@ -1425,68 +1453,109 @@ __device__ __forceinline__ void ms_fail(const MultiArgs &a, MultiShared &sh) {
     store_i(&a.ctl[0].err, 1);
 }
 
-// Rows j < E of an MFMA product's input from wavefront w = j % 4 (chunk c of 4 inputs in lane c % 64):
-// x = [first CA inputs; the rest], each chunk given by ld(j, c), then the row exponent and the digits
-// in the 16-row layout (k-block t, digit d at sq + t 2048 + d 1024, lane 16 g + j), zero up to KB
-// k-blocks. Returns false when a wait fails.
-template <typename LD>
-__device__ __forceinline__ bool rows_digits(int E, int CK, int KB, uint8_t *sq, MultiShared &sh, LD ld) {
+// Waits for N chunks of four tagged words at words + off[i] (bit i of need), all loads issued before the
+// first wait: a round trip between workgroups costs about a microsecond. x[i] gets the values.
+template <int N>
+__device__ __forceinline__ bool wait_chunks(const uint64_t *words, const uint32_t (&off)[N], uint32_t need,
+                                            const uint32_t (&tag)[N], v4f (&x)[N], const int32_t *err, uint64_t ticks) {
+    uint64_t w[N][4];
+    const uint64_t deadline = (uint64_t)wall_clock64() + ticks;
+    for (int round = 0; need; round++) {
+#pragma unroll
+        for (int i = 0; i < N; i++)
+            if (need >> i & 1) {
+#pragma unroll
+                for (int u = 0; u < 4; u++) w[i][u] = word_load(words + off[i] + u);
+            }
+#pragma unroll
+        for (int i = 0; i < N; i++)
+            if ((need >> i & 1) && (uint32_t)(w[i][0] >> 32) == tag[i] && (uint32_t)(w[i][1] >> 32) == tag[i] &&
+                (uint32_t)(w[i][2] >> 32) == tag[i] && (uint32_t)(w[i][3] >> 32) == tag[i]) {
+                x[i] = v4f{word_value(w[i][0]), word_value(w[i][1]), word_value(w[i][2]), word_value(w[i][3])};
+                need &= ~(1u << i);
+            }
+        if (need && (round & 15) == 15 && ((uint64_t)wall_clock64() > deadline || load_i(err) != 0)) return false;
+    }
+    return true;
+}
+
+// The exponents and digits of the wavefront's two streams' rows [first; second]: lane l holds chunks l +
+// 64 i of each half (CA and CB chunks, zero past them) (i < NC) of streams wave (xa[i]) and wave + 4 (xa[NC + i]), and
+// stream q is row q of the 16-row layout (digit_slot), zero
+// past the row up to KB k-blocks. Both rows in one stretch of code, so that their chains overlap.
+template <int NC>
+__device__ __forceinline__ void stream_digits(const v4f (&xa)[2 * NC], int CA, const v4f (&xb)[2 * NC], int CB, int KB,
+                                              uint8_t *sq, MultiShared &sh) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    bool ok = true;
-    for (int j = wave; j < E; j += RES_WAVES) {
-        v4f x[8];
+    int32_t e[2];
+#pragma unroll
+    for (int rr = 0; rr < 2; rr++) {
         uint32_t mx = 0;
 #pragma unroll
-        for (int q = 0; q < 8; q++) {
-            const int c = lane + 64 * q;
-            x[q] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-            if (c < CK) {
-                ok = ld(j, c, x[q]) && ok;
-                mx = max(mx, chunk_max(x[q]));
-            }
-        }
+        for (int i = 0; i < NC; i++) mx = max(mx, max(chunk_max(xa[NC * rr + i]), chunk_max(xb[NC * rr + i])));
         const uint32_t m = gemv::wave_max_u(mx);
-        const int32_t e = m == 0xffffffffu ? EXP_NONFINITE : row_exponent_of(__uint_as_float(m));
-#pragma unroll
-        for (int q = 0; q < 8; q++) {
-            const int c = lane + 64 * q;
-            if (c < KB * 16) {
-                uint32_t hi, lo;
-                digits4(x[q].x, x[q].y, x[q].z, x[q].w, e, hi, lo);
-                uint8_t *d = sq + (c >> 4) * 2048 + ((c & 15) >> 2) * 256 + j * 16 + (c & 3) * 4;
-                *reinterpret_cast<uint32_t *>(d) = hi;
-                *reinterpret_cast<uint32_t *>(d + 1024) = lo;
-            }
-        }
-        if (lane == 0) sh.erow[j] = e;
+        e[rr] = m == 0xffffffffu ? EXP_NONFINITE : row_exponent_of(__uint_as_float(m));
     }
-    return ok;
+    auto put = [&](int c, int rr, v4f v) {
+        uint32_t hi, lo;
+        digits4(v.x, v.y, v.z, v.w, e[rr], hi, lo);
+        uint8_t *d = sq + digit_chunk(c, wave + RES_WAVES * rr);
+        *reinterpret_cast<uint32_t *>(d) = hi;
+        *reinterpret_cast<uint32_t *>(d + 1024) = lo;
+    };
+#pragma unroll
+    for (int rr = 0; rr < 2; rr++) {
+#pragma unroll
+        for (int i = 0; i < NC; i++) {
+            const int c = lane + 64 * i;
+            if (c < CA) put(c, rr, xa[NC * rr + i]);
+            if (c < CB) put(CA + c, rr, xb[NC * rr + i]);
+        }
+        if (CA + CB + lane < KB * 16) put(CA + CB + lane, rr, v4f{0.0f, 0.0f, 0.0f, 0.0f});
+        if (lane == 0) sh.erow[wave + RES_WAVES * rr] = e[rr];
+    }
 }
 
-// The integer sums of the 16 rows in sq with one panel of KB k-blocks in LDS (one wavefront).
-__device__ __forceinline__ void rows_sums(const uint8_t *pw, int KB, const uint8_t *sq, gemv::v4i &hi, gemv::v4i &lo) {
-    const int lane = threadIdx.x & 63;
+// The integer sums of the streams' rows in sq with one panel of KB k-blocks in LDS, in the lanes of
+// wavefront 0: every wavefront takes k-blocks w, w + 4, ... and the sums meet in sh.part (exact, so the split
+// changes nothing). One barrier inside; the caller's next one frees sh.part.
+__device__ __forceinline__ void rows_sums(const uint8_t *pw, int KB, const uint8_t *sq, MultiShared &sh, gemv::v4i &hi,
+                                          gemv::v4i &lo) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     hi = gemv::v4i{0, 0, 0, 0};
     lo = gemv::v4i{0, 0, 0, 0};
-    for (int t = 0; t < KB; t++) {
-        const gemv::v4i ah = *reinterpret_cast<const gemv::v4i *>(sq + t * 2048 + lane * 16);
-        const gemv::v4i al = *reinterpret_cast<const gemv::v4i *>(sq + t * 2048 + 1024 + lane * 16);
-        const gemv::v4i wv = *reinterpret_cast<const gemv::v4i *>(pw + (size_t)t * 1024 + lane * 16);
-        hi = __builtin_amdgcn_mfma_i32_16x16x64_i8(ah, wv, hi, 0, 0, 0);
-        lo = __builtin_amdgcn_mfma_i32_16x16x64_i8(al, wv, lo, 0, 0, 0);
+    for (int t0 = wave; t0 < KB; t0 += 5 * RES_WAVES) {  // five k-blocks' operands before their MFMAs
+        gemv::v4i ah[5], al[5], wv[5];
+#pragma unroll
+        for (int u = 0; u < 5; u++) {
+            const int t = min(t0 + u * RES_WAVES, KB - 1);
+            ah[u] = *reinterpret_cast<const gemv::v4i *>(sq + digit_slot(t, lane >> 4, lane & 15));
+            al[u] = *reinterpret_cast<const gemv::v4i *>(sq + 1024 + digit_slot(t, lane >> 4, lane & 15));
+            wv[u] = *reinterpret_cast<const gemv::v4i *>(pw + (size_t)t * 1024 + lane * 16);
+        }
+#pragma unroll
+        for (int u = 0; u < 5; u++) {
+            if (t0 + u * RES_WAVES >= KB) break;
+            hi = __builtin_amdgcn_mfma_i32_16x16x64_i8(ah[u], wv[u], hi, 0, 0, 0);
+            lo = __builtin_amdgcn_mfma_i32_16x16x64_i8(al[u], wv[u], lo, 0, 0, 0);
+        }
+    }
+    if (wave && lane < 4 * MS_MAX) {  // rows 4 (lane / 16) + 0..3: the streams'
+        sh.part[wave - 1][0][lane] = hi;
+        sh.part[wave - 1][1][lane] = lo;
+    }
+    __syncthreads();
+    if (wave == 0 && lane < 4 * MS_MAX) {
+#pragma unroll
+        for (int w = 0; w < RES_WAVES - 1; w++) {
+            hi += sh.part[w][0][lane];
+            lo += sh.part[w][1][lane];
+        }
     }
 }
 
-// Waits for the four words of chunk c at p (the value of each word its float), tag tg.
-__device__ __forceinline__ bool wait_chunk(const uint64_t *p, uint32_t tg, const int32_t *err, uint64_t ticks, v4f &x) {
-    const uint64_t *pp[4] = {p, p + 1, p + 2, p + 3};
-    const uint32_t tag[4] = {tg, tg, tg, tg};
-    uint64_t w[4];
-    const bool ok = wait_words<4>(pp, 0xfu, tag, w, err, (uint64_t)wall_clock64() + ticks);
-    x = v4f{word_value(w[0]), word_value(w[1]), word_value(w[2]), word_value(w[3])};
-    return ok;
-}
-
+// L: the most LSTM layers (a.layers <= L); NC: the chunks of 4 inputs a lane holds of h (h <= 256 NC).
+template <int L, int NC>
 __global__ __launch_bounds__(RES_THREADS) void tdt_multi_kernel(MultiArgs a) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     __shared__ MultiShared sh;
@@ -1502,8 +1571,10 @@ __global__ __launch_bounds__(RES_THREADS) void tdt_multi_kernel(MultiArgs a) {
     const int32_t *err = &a.ctl[0].err;
     uint8_t *wj = lds;
     uint8_t *wl = wj + (size_t)a.JP * KBJ * 1024;
-    uint8_t *wp = wl + (size_t)a.layers * a.LP * KBL * 1024;
-    uint8_t *sq = wp + (size_t)a.PP * KBP * 1024;
+    // The projection's panels: their workgroups hold no others when the grid has room (qoff > 0).
+    const size_t upper = ((size_t)a.JP * KBJ + (size_t)a.layers * a.LP * KBL) * 1024, low = (size_t)a.PP * KBP * 1024;
+    uint8_t *wp = a.qoff ? lds : lds + upper;
+    uint8_t *sq = lds + (a.qoff ? max(upper, low) : upper + low);
     float *pin = reinterpret_cast<float *>(sq + (size_t)max(KBJ4, max(KBL, KBP)) * 2048);  // [M][h]
     float *hst = pin + (size_t)M * h;                                                       // [layers][M][LP 4]
     float *cst = hst + (size_t)a.layers * M * a.LP * 4;
@@ -1552,9 +1623,36 @@ __global__ __launch_bounds__(RES_THREADS) void tdt_multi_kernel(MultiArgs a) {
         sh.pin_n[tid] = TAG_NONE;
     }
     if (tid == 0) sh.abort = 0;
+    // Thread q's stream for the decider, read from the arguments once.
+    const int my_frames = a.frames[min(tid, M - 1)], my_cap = a.cap[min(tid, M - 1)];
+    int32_t *const my_tokens = a.tokens[min(tid, M - 1)];
     uint32_t s = a.ctl[0].step;
     const uint32_t s_end = s + (uint32_t)a.steps;
     const int CH = h >> 2;
+    // LSTM outputs of this wavefront's streams wave and wave + 4 (lane l: chunks l + 64 i), kept from
+    // the layer above's input or read while the decision is waited for, and the prediction counts they
+    // belong to: the recurrent halves then cost nothing when a token comes.
+    v4f hr[L][2 * NC];
+    uint32_t hv[L][2];
+#pragma unroll
+    for (int l = 0; l < L; l++) {
+#pragma unroll
+        for (int i = 0; i < 2 * NC; i++) hr[l][i] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+        hv[l][0] = hv[l][1] = TAG_NONE;
+    }
+    // The LSTM outputs of layer l under prediction count tag(q) of the streams q (of this wavefront's
+    // two) for which want(q) holds, into x.
+    auto read_h = [&](int l, auto want, auto tag_of, v4f (&x)[2 * NC]) -> bool {
+        uint32_t off[2 * NC], tag[2 * NC], need = 0;
+#pragma unroll
+        for (int i = 0; i < 2 * NC; i++) {
+            const int q = wave + RES_WAVES * (i / NC), qm = min(q, M - 1), c = lane + 64 * (i % NC);
+            tag[i] = tag_of(qm);
+            off[i] = (uint32_t)(((l * 2 + (int)(tag[i] & 1)) * M + qm) * h + 4 * min(c, CH - 1));
+            if (q < M && want(qm) && c < CH) need |= 1u << i;
+        }
+        return wait_chunks<2 * NC>(a.w_h + rc, off, need, tag, x, err, a.wait_ticks);
+    };
     __syncthreads();
 
     while (s != s_end) {
@@ -1566,62 +1664,89 @@ __global__ __launch_bounds__(RES_THREADS) void tdt_multi_kernel(MultiArgs a) {
             const int q = tid / S, r = tid % S;
             sh.live[tid] = q < M && !sh.st[q][4] && r < sh.st[q][3];
         }
+        __syncthreads();
         // ---- The joint over each stream's window rows.
         if (npj > 0) {
-            // The live streams' predictions (waited for only after they change).
-            for (int q = 0; q < M; q++) {
-                if (sh.st[q][4] || sh.pin_n[q] == sh.n[q]) continue;  // uniform
-                const uint32_t nq = sh.n[q];
-                for (int i = tid; i < h; i += RES_THREADS) {
-                    const uint64_t *p[1] = {a.w_pred + rc + ((size_t)(nq & 1) * M + q) * h + i};
-                    const uint32_t tag[1] = {nq};
-                    uint64_t w[1];
-                    if (!wait_words<1>(p, 1u, tag, w, err, (uint64_t)wall_clock64() + a.wait_ticks)) ms_fail(a, sh);
-                    pin[(size_t)q * h + i] = word_value(w[0]);
-                }
-                __syncthreads();
-                if (tid == 0) sh.pin_n[q] = nq;
-            }
-            __syncthreads();
-            if (sh.abort) break;
+            // The encoder rows of the slots, requested before the wait for the predictions.
+            v4f e[4][NC];
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                const int r = wave + 4 * j;  // the row slot
-                if (sh.live[r]) {
-                    const int q = r / S, rr = r % S, f = min(sh.st[q][0] + rr, a.frames[q] - 1);
-                    const float *er = a.enc[q] + (size_t)f * a.lde[q];
-                    const float *pr = pin + (size_t)q * h;
-                    v4f z[4];
-                    uint32_t mx = 0;
+                const int r = wave + 4 * j, q = r / S;
+                const bool lv = sh.live[r];
+                const int f = lv ? min(sh.st[q][0] + r % S, a.frames[q] - 1) : 0;
+                const float *er = lv ? a.enc[q] + (size_t)f * a.lde[q] : nullptr;
 #pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        const int c = lane + 64 * i;
-                        z[i] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-                        if (c < CH) {
-                            const v4f e = *reinterpret_cast<const v4f *>(er + 4 * c);
-                            const v4f pv = *reinterpret_cast<const v4f *>(pr + 4 * c);
-                            z[i].x = fmaxf(e.x + pv.x, 0.0f);
-                            z[i].y = fmaxf(e.y + pv.y, 0.0f);
-                            z[i].z = fmaxf(e.z + pv.z, 0.0f);
-                            z[i].w = fmaxf(e.w + pv.w, 0.0f);
-                            mx = max(mx, chunk_max(z[i]));
-                        }
-                    }
-                    const uint32_t m = gemv::wave_max_u(mx);
-                    const int32_t ex = m == 0xffffffffu ? EXP_NONFINITE : row_exponent_of(__uint_as_float(m));
-#pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        const int c = lane + 64 * i;
-                        if (c < KBJ4 * 16) {
-                            uint32_t hi, lo;
-                            digits4(z[i].x, z[i].y, z[i].z, z[i].w, ex, hi, lo);
-                            uint8_t *d = sq + (c >> 4) * 2048 + ((c & 15) >> 2) * 256 + r * 16 + (c & 3) * 4;
-                            *reinterpret_cast<uint32_t *>(d) = hi;
-                            *reinterpret_cast<uint32_t *>(d + 1024) = lo;
-                        }
-                    }
-                    if (lane == 0) sh.erow[r] = ex;
+                for (int i = 0; i < NC; i++) {
+                    const int c = lane + 64 * i;
+                    e[j][i] = *reinterpret_cast<const v4f *>(lv && c < CH ? er + 4 * c : gemv::ZERO_CHUNK);
                 }
+            }
+            // The live streams' predictions (waited for only after they change), all of them at once.
+            uint32_t off[NC * MS_MAX], tag[NC * MS_MAX], need = 0;
+            uint64_t w[NC * MS_MAX];
+            bool fresh = false;
+#pragma unroll
+            for (int q = 0; q < MS_MAX; q++) {
+                const int qm = min(q, M - 1);
+                const uint32_t nq = sh.n[qm];
+                const bool wanted = q < M && !sh.st[qm][4] && sh.pin_n[qm] != nq;
+                fresh = fresh || wanted;  // uniform
+#pragma unroll
+                for (int v = 0; v < NC; v++) {
+                    const int i = tid + RES_THREADS * v;
+                    off[NC * q + v] = ((nq & 1) * M + qm) * h + min(i, h - 1);
+                    tag[NC * q + v] = nq;
+                    if (wanted && i < h) need |= 1u << (NC * q + v);
+                }
+            }
+            if (fresh) {
+                if (!wait_offsets<NC * MS_MAX>(a.w_pred + rc, off, need, tag, w, err, (uint64_t)wall_clock64() + a.wait_ticks))
+                    ms_fail(a, sh);
+#pragma unroll
+                for (int q = 0; q < MS_MAX; q++)
+#pragma unroll
+                    for (int v = 0; v < NC; v++)
+                        if (need >> (NC * q + v) & 1) pin[(size_t)q * h + tid + RES_THREADS * v] = word_value(w[NC * q + v]);
+                __syncthreads();
+                if (sh.abort) break;
+                if (tid < M) sh.pin_n[tid] = sh.n[tid];  // read again only after the barriers below
+            }
+            // The digits of the four row slots of this wavefront in one stretch, so that their chains
+            // overlap; a slot without a frame gets digits of its stream's prediction, which nothing reads.
+            int32_t ex[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const float *pr = pin + (size_t)min((wave + 4 * j) / S, M - 1) * h;
+                uint32_t mx = 0;
+#pragma unroll
+                for (int i = 0; i < NC; i++) {
+                    const int c = lane + 64 * i;
+                    const v4f pv = *reinterpret_cast<const v4f *>(c < CH ? pr + 4 * c : pr);
+                    v4f &z = e[j][i];
+                    z.x = c < CH ? fmaxf(z.x + pv.x, 0.0f) : 0.0f;
+                    z.y = c < CH ? fmaxf(z.y + pv.y, 0.0f) : 0.0f;
+                    z.z = c < CH ? fmaxf(z.z + pv.z, 0.0f) : 0.0f;
+                    z.w = c < CH ? fmaxf(z.w + pv.w, 0.0f) : 0.0f;
+                    mx = max(mx, chunk_max(z));
+                }
+                const uint32_t m = gemv::wave_max_u(mx);
+                ex[j] = m == 0xffffffffu ? EXP_NONFINITE : row_exponent_of(__uint_as_float(m));
+            }
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const int r = wave + 4 * j;
+#pragma unroll
+                for (int i = 0; i < NC; i++) {
+                    const int c = lane + 64 * i;
+                    if (c < KBJ4 * 16) {
+                        uint32_t hi, lo;
+                        digits4(e[j][i].x, e[j][i].y, e[j][i].z, e[j][i].w, ex[j], hi, lo);
+                        uint8_t *d = sq + digit_chunk(c, r);
+                        *reinterpret_cast<uint32_t *>(d) = hi;
+                        *reinterpret_cast<uint32_t *>(d + 1024) = lo;
+                    }
+                }
+                if (lane == 0) sh.erow[r] = ex[j];
             }
             __syncthreads();
             Key mine[4], dmine[4];
@@ -1635,8 +1760,8 @@ __global__ __launch_bounds__(RES_THREADS) void tdt_multi_kernel(MultiArgs a) {
                     gemv::v4i ah[4], al[4], wv[4];
 #pragma unroll
                     for (int u = 0; u < 4; u++) {
-                        ah[u] = *reinterpret_cast<const gemv::v4i *>(sq + (t0 + u) * 2048 + lane * 16);
-                        al[u] = *reinterpret_cast<const gemv::v4i *>(sq + (t0 + u) * 2048 + 1024 + lane * 16);
+                        ah[u] = *reinterpret_cast<const gemv::v4i *>(sq + digit_slot(t0 + u, lane >> 4, j16));
+                        al[u] = *reinterpret_cast<const gemv::v4i *>(sq + 1024 + digit_slot(t0 + u, lane >> 4, j16));
                         wv[u] = *reinterpret_cast<const gemv::v4i *>(wb + (size_t)min(t0 + u, KBJ - 1) * 1024);
                     }
 #pragma unroll
@@ -1647,12 +1772,14 @@ __global__ __launch_bounds__(RES_THREADS) void tdt_multi_kernel(MultiArgs a) {
                 }
                 const int col = (pj0 + pi) * PANEL + j16;
                 const float sc = sh.js[pi * PANEL + j16], bs = sh.jbias[pi * PANEL + j16];
+                const bool fits = __all((int)dequant_fits(hi[0]) & (int)dequant_fits(hi[1]) &
+                                        (int)dequant_fits(hi[2]) & (int)dequant_fits(hi[3]));
 #pragma unroll
                 for (int v = 0; v < 4; v++) {
                     const int r = orow + v;
                     if (sh.live[r] && col < NJ) {
-                        float val = epilogue_vals(dequant(hi[v], lo[v], sh.erow[r], sc), true, bs, ACT_NONE, 1.0f,
-                                                  false, 0.0f);
+                        float val = epilogue_vals(dequant_w(hi[v], lo[v], sh.erow[r], sc, fits), true, bs, ACT_NONE,
+                                                  1.0f, false, 0.0f);
                         const bool voc = col < a.vocab;
                         const int idx = voc ? col : col - a.vocab;
                         if (idx == 0 && __builtin_isnan(val)) val = __builtin_inff();
@@ -1686,6 +1813,21 @@ __global__ __launch_bounds__(RES_THREADS) void tdt_multi_kernel(MultiArgs a) {
             word_store(a.w_part + ((size_t)par * TDT_ROWS + tid) * RES_MAX_GRID + b, tagged_key(x, s));
             if (bq >= jd0 && bq < jd0 + nd)
                 word_store(a.w_dur + ((size_t)par * TDT_ROWS + tid) * TDT_ROWS + (bq - jd0), tagged_key(xd, s));
+        }
+        // The LSTM outputs of the last prediction that no layer's input has brought (the top layer's, and
+        // every layer's at the start): this workgroup's next joint word, which the buffer's rewriting
+        // waits for, comes after them.
+        if (npl > 0) {
+            bool ok = true;
+#pragma unroll
+            for (int l = 0; l < L; l++) {
+                if (l >= a.layers) break;
+                auto want = [&](int q) { return !sh.st[q][4] && hv[l][q / RES_WAVES] != sh.n[q]; };
+                ok = read_h(l, want, [&](int q) { return sh.n[q]; }, hr[l]) && ok;
+#pragma unroll
+                for (int rr = 0; rr < 2; rr++) hv[l][rr] = sh.n[min(wave + RES_WAVES * rr, M - 1)];
+            }
+            if (!ok) ms_fail(a, sh);
         }
         // ---- The decisions: workgroup 0 gathers every slot's words (sixteen threads a slot) and walks
         // each stream's window.
@@ -1750,8 +1892,8 @@ __global__ __launch_bounds__(RES_THREADS) void tdt_multi_kernel(MultiArgs a) {
                     d[5] = 1;
                 } else {
                     const Walked wk = walk_window(sh.st[tid][0], sh.st[tid][3], sh.st[tid][1], sh.st[tid][2],
-                                                  sh.tok_s + tid * S, sh.dur_s + tid * S, a.blank, a.frames[tid],
-                                                  a.max_symbols, a.tokens[tid], a.cap[tid], true);
+                                                  sh.tok_s + tid * S, sh.dur_s + tid * S, a.blank, my_frames,
+                                                  a.max_symbols, my_tokens, my_cap, true);
                     d[0] = wk.t;
                     d[1] = wk.on;
                     d[2] = wk.ntok;
@@ -1784,58 +1926,77 @@ __global__ __launch_bounds__(RES_THREADS) void tdt_multi_kernel(MultiArgs a) {
             sh.st[tid][1] = sh.dec[tid][1];
             sh.st[tid][2] = sh.dec[tid][2];
             sh.st[tid][3] = sh.dec[tid][4];
-            sh.st[tid][4] = sh.dec[tid][5] || sh.dec[tid][0] >= a.frames[tid];
+            sh.st[tid][4] = sh.dec[tid][5] || sh.dec[tid][0] >= my_frames;
         }
         if (tid == 0) {
             int e = 0;
-            for (int q = 0; q < M; q++)
-                if (sh.dec[q][3] >= 0) sh.emit[e++] = q;
+            for (int q = 0; q < M; q++) e += sh.dec[q][3] >= 0;
             sh.nemit = e;
         }
         __syncthreads();
         s++;
-        const int E = sh.nemit;
-        if (E == 0) continue;
+        if (sh.nemit == 0) continue;
 
-        // ---- The prediction network for the E emitting streams, row j the j-th of them.
+        // ---- The prediction network for the emitting streams, stream q as row q (the other rows hold
+        // whatever digits were there and are not stored).
+        auto emits = [&](int q) { return sh.dec[q][3] >= 0; };
+        auto next_tag = [&](int q) { return sh.n[q] + 1; };
         bool stop = false;
-        for (int l = 0; l < a.layers && !stop; l++) {
+#pragma unroll
+        for (int l = 0; l < L; l++) {
+            if (l >= a.layers || stop) break;
             if (npl == 0) continue;
             const uint8_t *wlay = wl + (size_t)l * a.LP * KBL * 1024;
-            auto ld = [&](int j, int c, v4f &x) -> bool {
-                const int q = sh.emit[j];
-                const uint32_t nq = sh.n[q];
-                if (c < CH) {
-                    if (l == 0) {
-                        x = *reinterpret_cast<const v4f *>(a.emb + (size_t)sh.dec[q][3] * h + 4 * c);
-                        return true;
-                    }
-                    return wait_chunk(a.w_h + rc + (((size_t)(l - 1) * 2 + ((nq + 1) & 1)) * M + q) * h + 4 * c, nq + 1,
-                                      err, a.wait_ticks, x);
+            // [the embedding row or the layer below's new outputs; this layer's old outputs].
+            bool ok = true;
+            if (l == 0) {
+                v4f x[2 * NC];
+#pragma unroll
+                for (int i = 0; i < 2 * NC; i++) {
+                    const int q = min(wave + RES_WAVES * (i / NC), M - 1), c = lane + 64 * (i % NC), tok = sh.dec[q][3];
+                    x[i] = *reinterpret_cast<const v4f *>(c < CH && tok >= 0 ? a.emb + (size_t)tok * h + 4 * c
+                                                                             : gemv::ZERO_CHUNK);
                 }
-                return wait_chunk(a.w_h + rc + (((size_t)l * 2 + (nq & 1)) * M + q) * h + 4 * (c - CH), nq, err,
-                                  a.wait_ticks, x);
-            };
-            if (!rows_digits(E, 2 * CH, KBL, sq, sh, ld)) ms_fail(a, sh);
+                stream_digits<NC>(x, CH, hr[0], CH, KBL, sq, sh);
+            } else {
+                ok = read_h(l - 1, emits, next_tag, hr[l > 0 ? l - 1 : 0]);
+#pragma unroll
+                for (int rr = 0; rr < 2; rr++) {
+                    const int q = min(wave + RES_WAVES * rr, M - 1);
+                    hv[l > 0 ? l - 1 : 0][rr] = sh.n[q] + (emits(q) ? 1 : 0);
+                }
+                stream_digits<NC>(hr[l > 0 ? l - 1 : 0], CH, hr[l], CH, KBL, sq, sh);
+            }
+            if (!ok) ms_fail(a, sh);
             __syncthreads();
             if (sh.abort) {
                 stop = true;
                 break;
             }
-            for (int pi = wave; pi < npl; pi += RES_WAVES) {
+            for (int pi = 0; pi < npl; pi++) {
                 gemv::v4i hi, lo;
-                rows_sums(wlay + (size_t)pi * KBL * 1024, KBL, sq, hi, lo);
-                const int j16 = lane & 15, orow = (lane >> 4) * 4;
-                const float sc = sh.ls[l][pi * PANEL + j16], bs = sh.lbias[l][pi * PANEL + j16];
+                rows_sums(wlay + (size_t)pi * KBL * 1024, KBL, sq, sh, hi, lo);
+                if (wave == 0) {
+                    const int j16 = lane & 15, orow = (lane >> 4) * 4, k = j16 & 3;
+                    const float sc = sh.ls[l][pi * PANEL + j16], bs = sh.lbias[l][pi * PANEL + j16];
+                    const bool fits = __all((int)dequant_fits(hi[0]) & (int)dequant_fits(hi[1]) &
+                                            (int)dequant_fits(hi[2]) & (int)dequant_fits(hi[3]));
+                    // A quad of lanes holds a unit's four gates of four rows; lane k of it takes row k.
+                    float gi = 0.0f, gf = 0.0f, gg = 0.0f, go = 0.0f;
 #pragma unroll
-                for (int v = 0; v < 4; v++) {
-                    const int r = orow + v;
-                    const float val = epilogue_vals(dequant(hi[v], lo[v], sh.erow[min(r, E - 1)], sc), true, bs,
-                                                    ACT_NONE, 1.0f, false, 0.0f);
-                    const float gi = quad_lane<0>(val), gf = quad_lane<1>(val), gg = quad_lane<2>(val),
-                                go = quad_lane<3>(val);
-                    if (r < E && (j16 & 3) == 0) {
-                        const int q = sh.emit[r], ul = pi * 4 + (j16 >> 2), u = pl0 * 4 + ul;
+                    for (int v = 0; v < 4; v++) {
+                        const float val = epilogue_vals(dequant_w(hi[v], lo[v], sh.erow[orow + v], sc, fits), true, bs,
+                                                        ACT_NONE, 1.0f, false, 0.0f);
+                        const float q0 = quad_lane<0>(val), q1 = quad_lane<1>(val), q2 = quad_lane<2>(val),
+                                    q3 = quad_lane<3>(val);
+                        gi = k == v ? q0 : gi;
+                        gf = k == v ? q1 : gf;
+                        gg = k == v ? q2 : gg;
+                        go = k == v ? q3 : go;
+                    }
+                    const int q = orow + k;
+                    if (q < M && emits(q)) {
+                        const int ul = pi * 4 + (j16 >> 2), u = pl0 * 4 + ul;
                         const uint32_t nn = sh.n[q] + 1;
                         float *cs_ = cst + ((size_t)l * M + q) * U + ul, *hs_ = hst + ((size_t)l * M + q) * U + ul;
                         const float ig = sigmoid(gi), fg = sigmoid(gf), gt = tanhf(gg), og = sigmoid(go);
@@ -1846,41 +2007,42 @@ __global__ __launch_bounds__(RES_THREADS) void tdt_multi_kernel(MultiArgs a) {
                         word_store_all(a.w_h + (((size_t)l * 2 + (nn & 1)) * M + q) * h + u, a.cs, tagged(hn, nn));
                     }
                 }
+                __syncthreads();
             }
-            __syncthreads();
         }
         if (stop) break;
         if (npp > 0) {
-            auto ld = [&](int j, int c, v4f &x) -> bool {
-                const int q = sh.emit[j];
-                const uint32_t nn = sh.n[q] + 1;
-                return wait_chunk(a.w_h + rc + (((size_t)(a.layers - 1) * 2 + (nn & 1)) * M + q) * h + 4 * c, nn, err,
-                                  a.wait_ticks, x);
-            };
-            if (!rows_digits(E, CH, KBP, sq, sh, ld)) ms_fail(a, sh);
+            v4f x[2 * NC], none[2 * NC];
+#pragma unroll
+            for (int i = 0; i < 2 * NC; i++) x[i] = none[i] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+            if (!read_h(a.layers - 1, emits, next_tag, x)) ms_fail(a, sh);
+            stream_digits<NC>(x, CH, none, 0, KBP, sq, sh);
             __syncthreads();
             if (sh.abort) break;
-            for (int pi = wave; pi < npp; pi += RES_WAVES) {
+            for (int pi = 0; pi < npp; pi++) {
                 gemv::v4i hi, lo;
-                rows_sums(wp + (size_t)pi * KBP * 1024, KBP, sq, hi, lo);
-                const int j16 = lane & 15, orow = (lane >> 4) * 4, col = (pp0 + pi) * PANEL + j16;
-                const float sc = sh.ps[pi * PANEL + j16], bs = sh.pbias[pi * PANEL + j16];
+                rows_sums(wp + (size_t)pi * KBP * 1024, KBP, sq, sh, hi, lo);
+                if (wave == 0) {
+                    const int j16 = lane & 15, orow = (lane >> 4) * 4, col = (pp0 + pi) * PANEL + j16;
+                    const float sc = sh.ps[pi * PANEL + j16], bs = sh.pbias[pi * PANEL + j16];
+                    const bool fits = __all((int)dequant_fits(hi[0]) & (int)dequant_fits(hi[1]) &
+                                            (int)dequant_fits(hi[2]) & (int)dequant_fits(hi[3]));
 #pragma unroll
-                for (int v = 0; v < 4; v++) {
-                    const int r = orow + v;
-                    if (r < E && col < h) {
-                        const int q = sh.emit[r];
-                        const uint32_t nn = sh.n[q] + 1;
-                        const float val = epilogue_vals(dequant(hi[v], lo[v], sh.erow[r], sc), true, bs, ACT_NONE,
-                                                        1.0f, false, 0.0f);
-                        pst[(size_t)q * a.PP * PANEL + pi * PANEL + j16] = val;
-                        word_store_all(a.w_pred + ((size_t)(nn & 1) * M + q) * h + col, a.cs, tagged(val, nn));
+                    for (int v = 0; v < 4; v++) {
+                        const int q = orow + v;
+                        if (q < M && emits(q) && col < h) {
+                            const uint32_t nn = sh.n[q] + 1;
+                            const float val = epilogue_vals(dequant_w(hi[v], lo[v], sh.erow[q], sc, fits), true, bs,
+                                                            ACT_NONE, 1.0f, false, 0.0f);
+                            pst[(size_t)q * a.PP * PANEL + pi * PANEL + j16] = val;
+                            word_store_all(a.w_pred + ((size_t)(nn & 1) * M + q) * h + col, a.cs, tagged(val, nn));
+                        }
                     }
                 }
+                __syncthreads();
             }
-            __syncthreads();
         }
-        if (tid < E) sh.n[sh.emit[tid]]++;
+        if (tid < M && emits(tid)) sh.n[tid]++;
         __syncthreads();
     }
 
@@ -2146,9 +2308,16 @@ size_t tdt_multi_words(const TdtNet &net) { return RES_COPIES * multi_words_per_
 static size_t multi_lds(const TdtNet &net, const TdtPlan &p) {
     const size_t KBJ = net.joint->kb, KBL = net.lstm[0]->kb, KBP = net.proj->kb;
     const size_t M = TDT_MAX_STREAMS;
-    return ((size_t)p.JP * KBJ + net.layers * p.LP * KBL + (size_t)p.PP * KBP) * 1024 +
+    const size_t upper = (size_t)p.JP * KBJ + net.layers * p.LP * KBL, low = (size_t)p.PP * KBP;
+    return (p.qoff ? std::max(upper, low) : upper + low) * 1024 +
            std::max(((KBJ + 3) & ~(size_t)3), std::max(KBL, KBP)) * 2048 +
            (M * net.h + 2 * net.layers * M * p.LP * 4 + M * p.PP * PANEL) * sizeof(float);
+}
+
+static const void *multi_kernel(const TdtNet &net) {
+    static_assert(TDT_MAX_H <= 4 * 256, "four chunks per lane");
+    return net.layers <= 2 && net.h <= 3 * 256 ? reinterpret_cast<const void *>(&tdt_multi_kernel<2, 3>)
+                                               : reinterpret_cast<const void *>(&tdt_multi_kernel<TDT_MAX_LAYERS, 4>);
 }
 
 bool tdt_multi_plan(const TdtNet &net, TdtPlan &plan) {
@@ -2160,7 +2329,7 @@ bool tdt_multi_plan(const TdtNet &net, TdtPlan &plan) {
         hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess)
         return false;
     const size_t lds = multi_lds(net, plan);
-    const void *f = reinterpret_cast<const void *>(&tdt_multi_kernel);
+    const void *f = multi_kernel(net);
     hipFuncAttributes fa;
     if (hipFuncGetAttributes(&fa, f) != hipSuccess || lds + fa.sharedSizeBytes > (size_t)max_lds) return false;
     if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) return false;
@@ -2235,8 +2404,8 @@ hipError_t launch_tdt_multi(TdtCtl *ctl, const TdtNet &net, const TdtPlan &plan,
     a.steps = steps;
     a.wait_ticks = wait_ticks;
     void *args[] = {&a};
-    return hipLaunchCooperativeKernel(reinterpret_cast<const void *>(&tdt_multi_kernel), dim3((unsigned)plan.grid),
-                                      dim3(RES_THREADS), args, (unsigned)plan.mlds, s);
+    return hipLaunchCooperativeKernel(multi_kernel(net), dim3((unsigned)plan.grid), dim3(RES_THREADS), args,
+                                      (unsigned)plan.mlds, s);
 }
 
 }  // namespace tg

@@ -416,6 +416,42 @@ def test_multi_stream_decode_matches_each_stream(tk, orc, case):
     dec.close()
 
 
+# The multi-stream kernel's instances (up to two layers of at most 768 units, else), rows that end inside
+# a k-block, one to eight streams over the four wavefronts.
+MULTI_EDGES = [  # h, vocab, layers, frames per stream
+    (100, 70, 3, [20, 31, 5, 18, 26]),
+    (768, 90, 2, [9, 14, 11]),
+    (772, 90, 2, [12, 7, 10, 9, 11, 8, 13]),
+    (36, 50, 4, [40, 1]),
+    (192, 60, 2, [25, 19, 22, 30, 8, 27]),
+]
+
+
+@pytest.mark.parametrize("h,vocab,layers,frames", MULTI_EDGES)
+def test_multi_stream_decode_at_its_edges_is_each_stream_alone(tk, h, vocab, layers, frames):
+    """Tokens, position, state and prediction of every stream, bit for bit those of the single-stream
+    decode (which the other tests hold against the oracle), twice over from the states of the first."""
+    import torch
+
+    rng = np.random.default_rng(7 * h + layers)
+    net = tdt_network(rng, h, vocab, [0, 1, 2], layers=layers, max_symbols=3, blank_bias=2.0)
+    dec = upload(tk, net)
+    dev = lambda a: torch.from_numpy(a.copy()).cuda()  # noqa: E731
+    sd = [dev((0.3 * rng.standard_normal(layers * 2 * h)).astype(np.float32)) for _ in frames]
+    pd = [dev((0.3 * rng.standard_normal(h)).astype(np.float32)) for _ in frames]
+    s1, p1 = [t.clone() for t in sd], [t.clone() for t in pd]
+    for turn in range(2):
+        encs = [dev(rng.standard_normal((f, h)).astype(np.float32)) for f in frames]
+        say("multi-stream edges", h, vocab, layers, frames, turn)
+        got = dec.decode_streams(encs, sd, pd)
+        assert dec.last_resident == 2
+        for q, enc in enumerate(encs):
+            assert dec.decode(enc, s1[q], p1[q]) == got[q], q
+            assert torch.equal(sd[q].view(torch.int32), s1[q].view(torch.int32)), q
+            assert torch.equal(pd[q].view(torch.int32), p1[q].view(torch.int32)), q
+    dec.close()
+
+
 def test_multi_stream_decode_falls_back_and_refuses(tk, orc):
     """With the resident decode off the streams run one after another on the step kernels, with the
     same tokens; a stream past its frames takes no part; shared states are refused."""
