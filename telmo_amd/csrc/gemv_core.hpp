@@ -33,6 +33,7 @@ struct RowsIn {
 
 // Outputs stored to c (row stride ldc).
 struct StoreC {
+    static constexpr bool ROWS4 = false;
     float *c;
     size_t ldc;
     __device__ __forceinline__ void store(int r, int col, float v) { c[(size_t)r * ldc + col] = v; }
@@ -269,6 +270,8 @@ __device__ __forceinline__ void mfma_body_impl(const In &in, Out &out, int m, in
     const uint8_t *dp = sqa + (lane >> 4) * 256;
     int par = 0;
     for (; p < P; p += step) {
+        if constexpr (Out::ROWS4)
+            if (kw == 0) out.begin(orow, min(p * PANEL + ocol, N - 1), m);
         v4i acc_hi = {0, 0, 0, 0}, acc_lo = {0, 0, 0, 0};
         v4f accq = {0.0f, 0.0f, 0.0f, 0.0f};
         int dh[DOTR > 0 ? DOTR : 1], dl[DOTR > 0 ? DOTR : 1];
@@ -384,18 +387,20 @@ __device__ __forceinline__ void mfma_body_impl(const In &in, Out &out, int m, in
         }
         const int col = p * PANEL + ocol;
         if (col < N && kw == 0) {
+            float y[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
             for (int v = 0; v < 4; v++) {
-                if (orow + v < m) {
+                if (Out::ROWS4 || orow + v < m) {
                     float s;
                     if constexpr (Q8)
                         s = erow[v] == EXP_NONFINITE ? __builtin_nanf("") : __builtin_ldexpf(accq[v], -erow[v]);
                     else
                         s = dequant(acc_hi[v], acc_lo[v], erow[v], sc0);
-                    out.store(orow + v, col,
-                              epilogue_vals(s, bias != nullptr, bv0, act, escale, accumulate != 0, old0[v]));
+                    y[v] = epilogue_vals(s, bias != nullptr, bv0, act, escale, accumulate != 0, old0[v]);
+                    if constexpr (!Out::ROWS4) out.store(orow + v, col, y[v]);
                 }
             }
+            if constexpr (Out::ROWS4) out.store4(orow, col, y, m);
         }
     }
 }

@@ -42,11 +42,12 @@ __device__ __forceinline__ float widen_one(const uint8_t *__restrict__ wv, const
     }
 }
 
-// The accuracy guard's fix-up (RowGuard): the exact kernel's sums (one lane per output: flagged rows
-// are few) and epilogue for the flagged rows of a product the fast path has just written, over every output column. Workgroup (x, y) takes the
-// 64 columns 64 x .. and the rows of chunk y; its wavefronts read the chunk's flags 64 at a time and
-// take the flagged rows in turn (wavefront w the w-th, w + 4-th, ... of each group of 64). A flagged
-// row's old outputs come from save (kept by the quantiser) when the epilogue accumulates.
+// The accuracy guard's fix-up (RowGuard): the exact kernel's sums (one lane per output, since flagged
+// rows are few) and epilogue for the flagged rows of a product the fast path has just written, over
+// every output column. Workgroup (x, y) takes the 64 columns 64 x .. and the rows of chunk y; its
+// wavefronts read the chunk's flags 64 at a time and take the flagged rows in turn (wavefront w the
+// w-th, w + 4-th, ... of each group of 64). A flagged row's old outputs come from save (kept by the
+// quantiser) when the epilogue accumulates.
 __global__ __launch_bounds__(256) void exact_rows_kernel(const float *__restrict__ a, size_t lda, int m, int k,
                                                          const uint8_t *__restrict__ wv,
                                                          const float *__restrict__ scales, uint32_t prec, int N,

@@ -83,6 +83,7 @@ struct JointIn {
 // Joint outputs: per lane the best vocabulary entry of its four rows so far; the first logit and the
 // duration logits of each row go to extras (row r at r * TDT_EXTRA: first, then the durations).
 struct JointOut {
+    static constexpr bool ROWS4 = false;
     float *extras;
     int vocab;
     float bv[4];
@@ -128,21 +129,38 @@ __device__ __forceinline__ float quad_lane(float v) {
 }
 
 // LSTM outputs on interleaved rows: output col = 4 u + q is gate q (i, f, g, o) of unit u. The four
-// lanes of a quad hold one unit's gates for the same row; lane q = 0 applies the cell update
-// (src/parakeet.rs:1549-1562): c = f c + i g, h = o tanh(c), each product rounded before the sum.
+// lanes of a quad hold one unit's gates of the same four rows; lane k of it applies the cell update
+// (src/parakeet.rs:1549-1562) to row k: c = f c + i g, h = o tanh(c), each product rounded before the
+// sum. The old cells are requested before the products: with one lane updating the four rows in turn,
+// each read waiting behind the row before's stores, a layer of eight rows took 10.5 us.
 struct LstmOut {
+    static constexpr bool ROWS4 = true;
     const float *s_in;
     float *s_out;
     size_t width;
     int h, l;
-    __device__ __forceinline__ void store(int r, int col, float v) {
-        const float gi = quad_lane<0>(v), gf = quad_lane<1>(v), gg = quad_lane<2>(v), go = quad_lane<3>(v);
-        if ((col & 3) == 0) {
-            const size_t at = (size_t)r * width + (size_t)l * 2 * h + (col >> 2);
-            const float i = sigmoid(gi), f = sigmoid(gf), g = tanhf(gg), o = sigmoid(go);
-            const float c = f * s_in[at + h] + i * g;
-            s_out[at + h] = c;
-            s_out[at] = o * tanhf(c);
+    float c_old = 0.0f;
+    __device__ __forceinline__ size_t at(int row, int col) const {
+        return (size_t)row * width + (size_t)l * 2 * h + (col >> 2);
+    }
+    __device__ __forceinline__ void begin(int orow, int col, int m) {
+        const int row = orow + (col & 3);
+        c_old = s_in[at(row < m ? row : 0, col) + h];
+    }
+    __device__ __forceinline__ void store4(int orow, int col, const float (&v)[4], int m) {
+        const int k = col & 3, row = orow + k;
+        float gate[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const float g[4] = {quad_lane<0>(v[r]), quad_lane<1>(v[r]), quad_lane<2>(v[r]), quad_lane<3>(v[r])};
+#pragma unroll
+            for (int q = 0; q < 4; q++) gate[q] = k == r ? g[q] : gate[q];
+        }
+        if (row < m) {
+            const float i = sigmoid(gate[0]), f = sigmoid(gate[1]), g = tanhf(gate[2]), o = sigmoid(gate[3]);
+            const float c = f * c_old + i * g;
+            s_out[at(row, col) + h] = c;
+            s_out[at(row, col)] = o * tanhf(c);
         }
     }
 };
@@ -664,16 +682,6 @@ __device__ __forceinline__ bool wait_words(const uint64_t *const (&p)[N], uint32
     }
 }
 
-// Where the 16 hi digits of inputs 64 t + 16 g .. of row r sit in the 16-row digit layout (the lo digits
-// 1024 bytes on): k-block t's 2 KB, then 256 bytes per group g with the rows' 16 bytes permuted by (t, g),
-// so that the lanes of a wavefront writing one row's chunks (16 pairs of t and g) meet 16 bank groups
-// instead of one; the 16 rows that an MFMA operand read takes are all there either way.
-__device__ __forceinline__ int digit_slot(int t, int g, int r) {
-    return t * 2048 + g * 256 + ((r ^ (((t & 3) << 2) | g)) << 4);
-}
-// The four digits of chunk c (inputs 4 c ..) of row r.
-__device__ __forceinline__ int digit_chunk(int c, int r) { return digit_slot(c >> 4, (c >> 2) & 3, r) + (c & 3) * 4; }
-
 // wait_words for the words at base + off[i].
 template <int N>
 __device__ __forceinline__ bool wait_offsets(const uint64_t *base, const uint32_t (&off)[N], uint32_t need,
@@ -1006,7 +1014,7 @@ __global__ __launch_bounds__(RES_THREADS) void tdt_resident_kernel(ResArgs a) {
                         if (c < KBJ4 * 16) {  // zero digits past the row (z is 0 there)
                             uint32_t hi, lo;
                             digits4(z[i].x, z[i].y, z[i].z, z[i].w, ex, hi, lo);
-                            uint8_t *d = sq + digit_chunk(c, r);
+                            uint8_t *d = sq + (c >> 4) * 2048 + ((c & 15) >> 2) * 256 + r * 16 + (c & 3) * 4;
                             *reinterpret_cast<uint32_t *>(d) = hi;
                             *reinterpret_cast<uint32_t *>(d + 1024) = lo;
                         }
@@ -1038,9 +1046,9 @@ __global__ __launch_bounds__(RES_THREADS) void tdt_resident_kernel(ResArgs a) {
                         gemv::v4i H[2], L[2];
 #pragma unroll
                         for (int hh = 0; hh < 2; hh++) {
-                            const int off = off0 + hh * 512, dig = digit_slot(t, 2 * hh + (g >> 1), j16) + 8 * (g & 1);
-                            const long ah = *reinterpret_cast<const long *>(sq + dig);
-                            const long al = *reinterpret_cast<const long *>(sq + 1024 + dig);
+                            const int off = off0 + hh * 512;
+                            const long ah = *reinterpret_cast<const long *>(sq + t * 2048 + off);
+                            const long al = *reinterpret_cast<const long *>(sq + t * 2048 + 1024 + off);
                             const long wv = *reinterpret_cast<const long *>(wb + (size_t)t * 1024 + off);
                             H[hh] = __builtin_amdgcn_mfma_i32_16x16x32_i8(ah, wv, gemv::v4i{0, 0, 0, 0}, 0, 0, 0);
                             L[hh] = __builtin_amdgcn_mfma_i32_16x16x32_i8(al, wv, gemv::v4i{0, 0, 0, 0}, 0, 0, 0);
@@ -1063,8 +1071,8 @@ __global__ __launch_bounds__(RES_THREADS) void tdt_resident_kernel(ResArgs a) {
                         gemv::v4i ah[4], al[4], wv[4];
 #pragma unroll
                         for (int u = 0; u < 4; u++) {
-                            ah[u] = *reinterpret_cast<const gemv::v4i *>(sq + digit_slot(t0 + u, lane >> 4, j16));
-                            al[u] = *reinterpret_cast<const gemv::v4i *>(sq + 1024 + digit_slot(t0 + u, lane >> 4, j16));
+                            ah[u] = *reinterpret_cast<const gemv::v4i *>(sq + (t0 + u) * 2048 + lane * 16);
+                            al[u] = *reinterpret_cast<const gemv::v4i *>(sq + (t0 + u) * 2048 + 1024 + lane * 16);
                             wv[u] = *reinterpret_cast<const gemv::v4i *>(wb + (size_t)min(t0 + u, KBJ - 1) * 1024);
                         }
 #pragma unroll
@@ -1481,7 +1489,7 @@ __device__ __forceinline__ bool wait_chunks(const uint64_t *words, const uint32_
 
 // The exponents and digits of the wavefront's two streams' rows [first; second]: lane l holds chunks l +
 // 64 i of each half (CA and CB chunks, zero past them) (i < NC) of streams wave (xa[i]) and wave + 4 (xa[NC + i]), and
-// stream q is row q of the 16-row layout (digit_slot), zero
+// stream q is row q of the 16-row layout (k-block t, digit d at sq + t 2048 + d 1024, lane 16 g + q), zero
 // past the row up to KB k-blocks. Both rows in one stretch of code, so that their chains overlap.
 template <int NC>
 __device__ __forceinline__ void stream_digits(const v4f (&xa)[2 * NC], int CA, const v4f (&xb)[2 * NC], int CB, int KB,
@@ -1499,7 +1507,7 @@ __device__ __forceinline__ void stream_digits(const v4f (&xa)[2 * NC], int CA, c
     auto put = [&](int c, int rr, v4f v) {
         uint32_t hi, lo;
         digits4(v.x, v.y, v.z, v.w, e[rr], hi, lo);
-        uint8_t *d = sq + digit_chunk(c, wave + RES_WAVES * rr);
+        uint8_t *d = sq + (c >> 4) * 2048 + ((c & 15) >> 2) * 256 + (wave + RES_WAVES * rr) * 16 + (c & 3) * 4;
         *reinterpret_cast<uint32_t *>(d) = hi;
         *reinterpret_cast<uint32_t *>(d + 1024) = lo;
     };
@@ -1529,8 +1537,8 @@ __device__ __forceinline__ void rows_sums(const uint8_t *pw, int KB, const uint8
 #pragma unroll
         for (int u = 0; u < 5; u++) {
             const int t = min(t0 + u * RES_WAVES, KB - 1);
-            ah[u] = *reinterpret_cast<const gemv::v4i *>(sq + digit_slot(t, lane >> 4, lane & 15));
-            al[u] = *reinterpret_cast<const gemv::v4i *>(sq + 1024 + digit_slot(t, lane >> 4, lane & 15));
+            ah[u] = *reinterpret_cast<const gemv::v4i *>(sq + t * 2048 + lane * 16);
+            al[u] = *reinterpret_cast<const gemv::v4i *>(sq + t * 2048 + 1024 + lane * 16);
             wv[u] = *reinterpret_cast<const gemv::v4i *>(pw + (size_t)t * 1024 + lane * 16);
         }
 #pragma unroll
@@ -1741,7 +1749,7 @@ __global__ __launch_bounds__(RES_THREADS) void tdt_multi_kernel(MultiArgs a) {
                     if (c < KBJ4 * 16) {
                         uint32_t hi, lo;
                         digits4(e[j][i].x, e[j][i].y, e[j][i].z, e[j][i].w, ex[j], hi, lo);
-                        uint8_t *d = sq + digit_chunk(c, r);
+                        uint8_t *d = sq + (c >> 4) * 2048 + ((c & 15) >> 2) * 256 + r * 16 + (c & 3) * 4;
                         *reinterpret_cast<uint32_t *>(d) = hi;
                         *reinterpret_cast<uint32_t *>(d + 1024) = lo;
                     }
@@ -1760,8 +1768,8 @@ __global__ __launch_bounds__(RES_THREADS) void tdt_multi_kernel(MultiArgs a) {
                     gemv::v4i ah[4], al[4], wv[4];
 #pragma unroll
                     for (int u = 0; u < 4; u++) {
-                        ah[u] = *reinterpret_cast<const gemv::v4i *>(sq + digit_slot(t0 + u, lane >> 4, j16));
-                        al[u] = *reinterpret_cast<const gemv::v4i *>(sq + 1024 + digit_slot(t0 + u, lane >> 4, j16));
+                        ah[u] = *reinterpret_cast<const gemv::v4i *>(sq + (t0 + u) * 2048 + lane * 16);
+                        al[u] = *reinterpret_cast<const gemv::v4i *>(sq + (t0 + u) * 2048 + 1024 + lane * 16);
                         wv[u] = *reinterpret_cast<const gemv::v4i *>(wb + (size_t)min(t0 + u, KBJ - 1) * 1024);
                     }
 #pragma unroll
