@@ -665,6 +665,18 @@ __device__ __forceinline__ int sum_groups(int v) {
     return (int)(b[0] + b[1]);
 }
 
+// The better of x over lanes l, l ^ 16, l ^ 32, l ^ 48.
+__device__ __forceinline__ Key fold_groups(Key x) {
+    const auto k16 = __builtin_amdgcn_permlane16_swap(x.k, x.k, false, false);
+    const auto i16 = __builtin_amdgcn_permlane16_swap(x.i, x.i, false, false);
+    const Key a{k16[0], i16[0]}, b{k16[1], i16[1]};
+    x = better(a, b) ? a : b;
+    const auto k32 = __builtin_amdgcn_permlane32_swap(x.k, x.k, false, false);
+    const auto i32 = __builtin_amdgcn_permlane32_swap(x.i, x.i, false, false);
+    const Key c{k32[0], i32[0]}, d{k32[1], i32[1]};
+    return better(c, d) ? c : d;
+}
+
 // Waits until word i (bit i of need) carries tag[i], reloading the words still pending each round.
 // False when the deadline passes or another workgroup has set the error flag.
 template <int N>
@@ -724,7 +736,7 @@ __device__ __forceinline__ void copy_panels(uint8_t *dst, const ResMat &m, int p
 
 // The LDS of a resident workgroup besides its panels.
 struct ResShared {
-    float js[RES_MAX_PANELS * PANEL], jbias[RES_MAX_PANELS * PANEL];
+    __attribute__((aligned(16))) float js[RES_MAX_PANELS * PANEL], jbias[RES_MAX_PANELS * PANEL];
     float ps[RES_MAX_PANELS * PANEL], pbias[RES_MAX_PANELS * PANEL], pst[RES_MAX_PANELS * PANEL];
     float ls[TDT_MAX_LAYERS][RES_MAX_PANELS * PANEL], lbias[TDT_MAX_LAYERS][RES_MAX_PANELS * PANEL];
     float hst[TDT_MAX_LAYERS][RES_MAX_PANELS * 4], cst[TDT_MAX_LAYERS][RES_MAX_PANELS * 4];
@@ -1023,15 +1035,15 @@ __global__ __launch_bounds__(RES_THREADS) void tdt_resident_kernel(ResArgs a) {
                 }
             }
             __syncthreads();
-            // Wavefront w scores panels w, w + 4, ... of this workgroup: element v of lane l is row
-            // 4 (l / 16) + v, column l % 16. Each row keeps its best vocabulary entry and its best
+            // Wavefront w scores panels w, w + 4, ... of this workgroup, the weights as the first operand:
+            // element v of lane l is row l % 16, column 4 (l / 16) + v, so a row's best entries meet over
+            // a lane's four columns and then four lanes (with the rows first, over sixteen lanes for
+            // each of a lane's four rows: 60 s decoded 5940 us, so 5693). Each row keeps its best vocabulary entry and its best
             // duration entry (index d for column vocab + d). A NaN first logit (column 0) is never
             // beaten in the reference's argmax: it enters as (+inf, 0), which nothing comes before;
             // a NaN first duration logit likewise.
-            Key mine[4], dmine[4];
-#pragma unroll
-            for (int v = 0; v < 4; v++) mine[v] = dmine[v] = Key{0u, 0xffffffffu};
-            const int orow = (lane >> 4) * 4, j16 = lane & 15;
+            Key mine{0u, 0xffffffffu}, dmine{0u, 0xffffffffu};
+            const int c4 = (lane >> 4) * 4, j16 = lane & 15;
             for (int pi = wave; pi < npj; pi += RES_WAVES) {
                 gemv::v4i hi = {0, 0, 0, 0}, lo = {0, 0, 0, 0};
                 float fq[4] = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -1040,7 +1052,7 @@ __global__ __launch_bounds__(RES_THREADS) void tdt_resident_kernel(ResArgs a) {
                     // lane 16 (2 hh + g / 2) + x, the same inputs for the digits and the weights. Both
                     // halves' MFMAs are issued before their folds, which run in block order.
                     const uint8_t *wb = wj + (size_t)pi * KBJ * 1024;
-                    const float *ds = qsj + (size_t)pi * NBJ * PANEL + j16;
+                    const float *ds = qsj + (size_t)pi * NBJ * PANEL + c4;
                     const int g = lane >> 4, off0 = (16 * (g >> 1) + j16) * 16 + 8 * (g & 1);
                     for (int t = 0; t < KBJ; t++) {
                         gemv::v4i H[2], L[2];
@@ -1050,16 +1062,16 @@ __global__ __launch_bounds__(RES_THREADS) void tdt_resident_kernel(ResArgs a) {
                             const long ah = *reinterpret_cast<const long *>(sq + t * 2048 + off);
                             const long al = *reinterpret_cast<const long *>(sq + t * 2048 + 1024 + off);
                             const long wv = *reinterpret_cast<const long *>(wb + (size_t)t * 1024 + off);
-                            H[hh] = __builtin_amdgcn_mfma_i32_16x16x32_i8(ah, wv, gemv::v4i{0, 0, 0, 0}, 0, 0, 0);
-                            L[hh] = __builtin_amdgcn_mfma_i32_16x16x32_i8(al, wv, gemv::v4i{0, 0, 0, 0}, 0, 0, 0);
+                            H[hh] = __builtin_amdgcn_mfma_i32_16x16x32_i8(wv, ah, gemv::v4i{0, 0, 0, 0}, 0, 0, 0);
+                            L[hh] = __builtin_amdgcn_mfma_i32_16x16x32_i8(wv, al, gemv::v4i{0, 0, 0, 0}, 0, 0, 0);
                         }
 #pragma unroll
                         for (int hh = 0; hh < 2; hh++) {
                             const int bk = 2 * t + hh;
                             if (bk < NBJ) {
-                                const float d = ds[bk * PANEL];
+                                const v4f d = *reinterpret_cast<const v4f *>(ds + bk * PANEL);
 #pragma unroll
-                                for (int v = 0; v < 4; v++) fq[v] = __builtin_fmaf(d, (float)(H[hh][v] * 256 + L[hh][v]), fq[v]);
+                                for (int v = 0; v < 4; v++) fq[v] = __builtin_fmaf(d[v], (float)(H[hh][v] * 256 + L[hh][v]), fq[v]);
                             }
                         }
                     }
@@ -1077,42 +1089,39 @@ __global__ __launch_bounds__(RES_THREADS) void tdt_resident_kernel(ResArgs a) {
                         }
 #pragma unroll
                         for (int u = 0; u < 4; u++) {
-                            hi = __builtin_amdgcn_mfma_i32_16x16x64_i8(ah[u], wv[u], hi, 0, 0, 0);
-                            lo = __builtin_amdgcn_mfma_i32_16x16x64_i8(al[u], wv[u], lo, 0, 0, 0);
+                            hi = __builtin_amdgcn_mfma_i32_16x16x64_i8(wv[u], ah[u], hi, 0, 0, 0);
+                            lo = __builtin_amdgcn_mfma_i32_16x16x64_i8(wv[u], al[u], lo, 0, 0, 0);
                         }
                     }
                 }
-                const int col = (pj0 + pi) * PANEL + j16;
-                const float sc = sh.js[pi * PANEL + j16], bs = sh.jbias[pi * PANEL + j16];
+                const v4f sc = *reinterpret_cast<const v4f *>(sh.js + pi * PANEL + c4);
+                const v4f bs = *reinterpret_cast<const v4f *>(sh.jbias + pi * PANEL + c4);
                 const bool fits = __all((int)dequant_fits(hi[0]) & (int)dequant_fits(hi[1]) &
                                         (int)dequant_fits(hi[2]) & (int)dequant_fits(hi[3]));
+                const int32_t er = sh.erow[j16];
 #pragma unroll
                 for (int v = 0; v < 4; v++) {
-                    const int r = orow + v;
-                    if (r < rows && col < NJ) {
-                        const int32_t er = sh.erow[r];
+                    const int col = (pj0 + pi) * PANEL + c4 + v;
+                    if (j16 < rows && col < NJ) {
                         const float dq = Q8 ? (er == EXP_NONFINITE ? __builtin_nanf("") : __builtin_ldexpf(fq[v], -er))
-                                            : dequant_w(hi[v], lo[v], er, sc, fits);
-                        float val = epilogue_vals(dq, true, bs, ACT_NONE, 1.0f, false, 0.0f);
+                                            : dequant_w(hi[v], lo[v], er, sc[v], fits);
+                        float val = epilogue_vals(dq, true, bs[v], ACT_NONE, 1.0f, false, 0.0f);
                         const bool voc = col < a.vocab;
                         const int idx = voc ? col : col - a.vocab;
                         if (idx == 0 && __builtin_isnan(val)) val = __builtin_inff();
                         // A lane meets its columns in increasing order: the strictly larger wins.
                         const uint32_t key = order_key(val);
-                        Key &m = voc ? mine[v] : dmine[v];
+                        Key &m = voc ? mine : dmine;
                         if (key > m.k) m = Key{key, (uint32_t)idx};
                     }
                 }
             }
             const bool has_dur = bq >= jd0 && bq < jd0 + nd;  // uniform: only these hold duration columns
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                mine[v] = fold16(mine[v]);
-                if (has_dur) dmine[v] = fold16(dmine[v]);
-                if (j16 == 0) {
-                    sh.red[wave][orow + v] = mine[v];
-                    sh.dred[wave][orow + v] = dmine[v];
-                }
+            mine = fold_groups(mine);
+            if (has_dur) dmine = fold_groups(dmine);
+            if (lane < TDT_ROWS) {
+                sh.red[wave][lane] = mine;
+                sh.dred[wave][lane] = dmine;
             }
         }
         __syncthreads();
@@ -1439,7 +1448,7 @@ struct MultiArgs {
 };
 
 struct MultiShared {
-    float js[RES_MAX_PANELS * PANEL], jbias[RES_MAX_PANELS * PANEL];
+    __attribute__((aligned(16))) float js[RES_MAX_PANELS * PANEL], jbias[RES_MAX_PANELS * PANEL];
     float ps[RES_MAX_PANELS * PANEL], pbias[RES_MAX_PANELS * PANEL];
     float ls[TDT_MAX_LAYERS][RES_MAX_PANELS * PANEL], lbias[TDT_MAX_LAYERS][RES_MAX_PANELS * PANEL];
     Key red[RES_WAVES][TDT_ROWS], dred[RES_WAVES][TDT_ROWS];
@@ -1757,10 +1766,8 @@ __global__ __launch_bounds__(RES_THREADS) void tdt_multi_kernel(MultiArgs a) {
                 if (lane == 0) sh.erow[r] = ex[j];
             }
             __syncthreads();
-            Key mine[4], dmine[4];
-#pragma unroll
-            for (int v = 0; v < 4; v++) mine[v] = dmine[v] = Key{0u, 0xffffffffu};
-            const int orow = (lane >> 4) * 4, j16 = lane & 15;
+            Key mine{0u, 0xffffffffu}, dmine{0u, 0xffffffffu};
+            const int c4 = (lane >> 4) * 4, j16 = lane & 15;
             for (int pi = wave; pi < npj; pi += RES_WAVES) {
                 gemv::v4i hi = {0, 0, 0, 0}, lo = {0, 0, 0, 0};
                 const uint8_t *wb = wj + (size_t)pi * KBJ * 1024 + lane * 16;
@@ -1774,38 +1781,37 @@ __global__ __launch_bounds__(RES_THREADS) void tdt_multi_kernel(MultiArgs a) {
                     }
 #pragma unroll
                     for (int u = 0; u < 4; u++) {
-                        hi = __builtin_amdgcn_mfma_i32_16x16x64_i8(ah[u], wv[u], hi, 0, 0, 0);
-                        lo = __builtin_amdgcn_mfma_i32_16x16x64_i8(al[u], wv[u], lo, 0, 0, 0);
+                        hi = __builtin_amdgcn_mfma_i32_16x16x64_i8(wv[u], ah[u], hi, 0, 0, 0);
+                        lo = __builtin_amdgcn_mfma_i32_16x16x64_i8(wv[u], al[u], lo, 0, 0, 0);
                     }
                 }
-                const int col = (pj0 + pi) * PANEL + j16;
-                const float sc = sh.js[pi * PANEL + j16], bs = sh.jbias[pi * PANEL + j16];
+                const v4f sc = *reinterpret_cast<const v4f *>(sh.js + pi * PANEL + c4);
+                const v4f bs = *reinterpret_cast<const v4f *>(sh.jbias + pi * PANEL + c4);
                 const bool fits = __all((int)dequant_fits(hi[0]) & (int)dequant_fits(hi[1]) &
                                         (int)dequant_fits(hi[2]) & (int)dequant_fits(hi[3]));
+                const int32_t er = sh.erow[j16];
+                const bool live = sh.live[j16];
 #pragma unroll
                 for (int v = 0; v < 4; v++) {
-                    const int r = orow + v;
-                    if (sh.live[r] && col < NJ) {
-                        float val = epilogue_vals(dequant_w(hi[v], lo[v], sh.erow[r], sc, fits), true, bs, ACT_NONE,
-                                                  1.0f, false, 0.0f);
+                    const int col = (pj0 + pi) * PANEL + c4 + v;
+                    if (live && col < NJ) {
+                        float val = epilogue_vals(dequant_w(hi[v], lo[v], er, sc[v], fits), true, bs[v], ACT_NONE, 1.0f,
+                                                  false, 0.0f);
                         const bool voc = col < a.vocab;
                         const int idx = voc ? col : col - a.vocab;
                         if (idx == 0 && __builtin_isnan(val)) val = __builtin_inff();
                         const uint32_t key = order_key(val);
-                        Key &m = voc ? mine[v] : dmine[v];
+                        Key &m = voc ? mine : dmine;
                         if (key > m.k) m = Key{key, (uint32_t)idx};
                     }
                 }
             }
             const bool has_dur = bq >= jd0 && bq < jd0 + nd;
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                mine[v] = fold16(mine[v]);
-                if (has_dur) dmine[v] = fold16(dmine[v]);
-                if (j16 == 0) {
-                    sh.red[wave][orow + v] = mine[v];
-                    sh.dred[wave][orow + v] = dmine[v];
-                }
+            mine = fold_groups(mine);
+            if (has_dur) dmine = fold_groups(dmine);
+            if (lane < TDT_ROWS) {
+                sh.red[wave][lane] = mine;
+                sh.dred[wave][lane] = dmine;
             }
         }
         __syncthreads();
