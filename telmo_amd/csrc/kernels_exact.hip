@@ -120,17 +120,18 @@ __device__ __forceinline__ const void *scalar(const void *p) {
     return reinterpret_cast<const void *>(((uint64_t)hi << 32) | lo);
 }
 // Each lane's 16 (or 4) bytes to LDS at lds + 16 (4) * lane, lds wave-uniform: from base + voff (a
-// wave-uniform base, the lane's byte offset) or from the lane's address.
+// wave-uniform base, the lane's byte offset) or from the lane's address. A copy reads M0 without an
+// interlock: one wait state after the scalar write (the compiler adds none inside an asm text).
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
 __device__ __forceinline__ void copy16(const void *base, uint32_t voff, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(scalar(base)) : "memory", "m0");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(scalar(base)) : "memory", "m0");
 }
 __device__ __forceinline__ void copy4(const void *base, uint32_t voff, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds), "v"(voff), "s"(scalar(base)) : "memory", "m0");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds), "v"(voff), "s"(scalar(base)) : "memory", "m0");
 }
 __device__ __forceinline__ void copy4_lanes(const void *p, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, off" ::"s"(lds), "v"(p) : "memory", "m0");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(lds), "v"(p) : "memory", "m0");
 }
 #pragma clang diagnostic pop
 // Waits until at most `ahead` stages of CPW copies are on the way (ahead <= A). Waiting for fewer

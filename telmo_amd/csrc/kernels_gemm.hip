@@ -662,11 +662,12 @@ __device__ __forceinline__ uint32_t lds_address(const void *p) {
 // 64 lanes x 16 bytes from base + voff (a wave-uniform base address in scalar registers plus each
 // lane's byte offset) to LDS at lds (the wave-uniform LDS address; lane l's bytes land at lds +
 // 16 l when voff = 16 l). M0 holds the LDS address; it is set before every copy and nothing else
-// here uses it.
+// here uses it. A copy reads M0 without an interlock and needs one wait state after the scalar
+// write, which the compiler does not add inside an asm text: hence the s_nop.
 __device__ __forceinline__ void copy_to_lds_s(const uint8_t *base, uint32_t voff, uint32_t lds) {
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(base) : "memory", "m0");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(base) : "memory", "m0");
 #pragma clang diagnostic pop
 }
 
@@ -911,7 +912,7 @@ hipError_t launch_lds(const uint8_t *qf, const int32_t *exps, size_t m, const De
 __device__ __forceinline__ void copy_dword_to_lds_s(const uint8_t *base, uint32_t voff, uint32_t lds) {
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds), "v"(voff), "s"(base) : "memory", "m0");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds), "v"(voff), "s"(base) : "memory", "m0");
 #pragma clang diagnostic pop
 }
 
