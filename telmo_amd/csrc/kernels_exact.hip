@@ -121,14 +121,16 @@ __device__ __forceinline__ const void *scalar(const void *p) {
 }
 // Each lane's 16 (or 4) bytes to LDS at lds + 16 (4) * lane, lds wave-uniform: from base + voff (a
 // wave-uniform base, the lane's byte offset) or from the lane's address. A copy reads M0 without an
-// interlock: one wait state after the scalar write (the compiler adds none inside an asm text).
+// interlock, one wait state after a scalar write, and the base's scalar registers five after a vector
+// one: scalar()'s v_readfirstlane, or the v_readlane of a spilled register. The compiler adds no wait
+// states inside an asm text, so the texts hold them (s_mov counts as one of the five).
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
 __device__ __forceinline__ void copy16(const void *base, uint32_t voff, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(scalar(base)) : "memory", "m0");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(scalar(base)) : "memory", "m0");
 }
 __device__ __forceinline__ void copy4(const void *base, uint32_t voff, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds), "v"(voff), "s"(scalar(base)) : "memory", "m0");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tglobal_load_lds_dword %1, %2" ::"s"(lds), "v"(voff), "s"(scalar(base)) : "memory", "m0");
 }
 __device__ __forceinline__ void copy4_lanes(const void *p, uint32_t lds) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(lds), "v"(p) : "memory", "m0");

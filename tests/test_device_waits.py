@@ -1,10 +1,12 @@
 """Wait states before the copies from global memory straight into LDS, in the built library's code.
 
 The copies are written in inline assembly, which the compiler's hazard recogniser does not look into, and
-M0, the LDS address, is read without an interlock: it needs one wait state after a scalar instruction has
-written it (AMD Instinct MI300 instruction set architecture, "Manually inserted wait states"). Each
-instruction between is one wait state and s_nop N is N + 1. The check reads the gfx950 code of the library
-that was built here and walks back from every copy along every path."""
+two of their operands are read without an interlock (AMD Instinct MI300 instruction set architecture,
+"Manually inserted wait states"): M0, the LDS address, needs one wait state after a scalar instruction has
+written it, and the scalar registers of the global address need five after a vector instruction (a
+v_readfirstlane_b32, or the v_readlane_b32 of a spilled register) has. Each instruction between is one
+wait state and s_nop N is N + 1. The check reads the gfx950 code of the library that was built here and
+walks back from every copy along every path."""
 import os
 import re
 import subprocess
@@ -17,11 +19,33 @@ OBJDUMP = os.environ.get("LLVM_OBJDUMP", "/opt/rocm/llvm/bin/llvm-objdump")
 LINE = re.compile(r"^\t(?P<text>\S.*?)\s*// (?P<at>[0-9A-F]+):.*?(?:<(?P<sym>[^>+]+)\+0x(?P<off>[0-9a-f]+)>)?$")
 SYMBOL = re.compile(r"^(?P<at>[0-9a-f]+) <(?P<name>.+)>:$")
 COPY = re.compile(r"(global|buffer|scratch)_load_.*\blds\b|(global|scratch)_load_lds_")
-STATES = 1  # the most that a write of an operand needs
+STATES = 5  # the most that a write of an operand needs
+
+
+def sgprs(text):
+    """The scalar registers that an operand text names, vcc as "vcc"."""
+    found = set(re.findall(r"\bvcc\b", text))
+    found.update(int(n) for n in re.findall(r"\bs(\d+)\b", text))
+    for lo, hi in re.findall(r"\bs\[(\d+):(\d+)\]", text):
+        found.update(range(int(lo), int(hi) + 1))
+    return found
+
+
+def written(text):
+    """The scalar registers that a vector instruction writes (its scalar destination operands)."""
+    name, _, rest = text.partition(" ")
+    operands = re.findall(r"[^\s,\[]+(?:\[[^\]]*\])?", rest)
+    found = sgprs(operands[0]) if operands else set()
+    # The carry-outs and div_scale's flag are second destinations.
+    if re.match(r"v_(add|sub|subrev|addc|subb|subbrev)_co_u32|v_div_scale|v_mad_[iu]64", name) and len(operands) > 1:
+        found |= sgprs(operands[1])
+    return found
 
 
 def too_early(text, states, copy):
     """Whether `text`, `states` wait states before `copy`, writes an operand that needs more."""
+    if text.startswith("v_"):
+        return states < 5 and bool(written(text) & sgprs(copy))
     return states < 1 and re.match(r"s_\S+ m0,", text) is not None
 
 
@@ -78,6 +102,17 @@ def test_the_check_finds_an_early_lds_address():
     loop = dump("s_nop 0", "s_nop 0", copy, "s_branch 65533")
     loop[-1] += " <kernel+0x8>"
     assert not hazards(loop)[0]
+
+
+def test_the_check_finds_an_early_base():
+    copy = "global_load_lds_dwordx4 v4, s[30:31]"
+    assert hazards(dump("v_readfirstlane_b32 s31, v2", "s_mov_b32 m0, s5", "s_nop 2", copy))[0]
+    assert not hazards(dump("v_readfirstlane_b32 s31, v2", "s_mov_b32 m0, s5", "s_nop 3", copy))[0]
+    assert not hazards(dump("v_readfirstlane_b32 s32, v2", "s_mov_b32 m0, s5", "s_nop 0", copy))[0]
+    assert hazards(dump("v_add_co_u32_e64 v1, s[30:31], v2, v3", "s_mov_b32 m0, s5", "s_nop 0", copy))[0]
+    loop = dump("s_nop 0", "s_nop 0", copy, "v_cmp_lt_i32_e64 s[30:31], v2, v3", "s_cbranch_scc1 65532")
+    loop[-1] += " <kernel+0x4>"
+    assert hazards(loop)[0]
 
 
 def test_copies_into_lds_wait_for_their_operands(tmp_path):
