@@ -1461,7 +1461,6 @@ struct MultiShared {
     uint32_t n[MS_MAX], pin_n[MS_MAX];
     int dec[MS_MAX][RES_DEC];
     int nemit;
-    __attribute__((aligned(16))) gemv::v4i part[RES_WAVES - 1][2][4 * MS_MAX];  // rows_sums' partial sums
     int abort;
 };
 
@@ -1534,10 +1533,14 @@ __device__ __forceinline__ void stream_digits(const v4f (&xa)[2 * NC], int CA, c
 }
 
 // The integer sums of the streams' rows in sq with one panel of KB k-blocks in LDS, in the lanes of
-// wavefront 0: every wavefront takes k-blocks w, w + 4, ... and the sums meet in sh.part (exact, so the split
-// changes nothing). One barrier inside; the caller's next one frees sh.part.
-__device__ __forceinline__ void rows_sums(const uint8_t *pw, int KB, const uint8_t *sq, MultiShared &sh, gemv::v4i &hi,
-                                          gemv::v4i &lo) {
+// wavefront 0: every wavefront takes k-blocks w, w + 4, ... and the sums meet in LDS (exact, so the split
+// changes nothing). They take no LDS of their own, which would cost networks near the limit this
+// kernel: wavefront w's go to the rows from MS_MAX on of k-block w (digit 0: hi, digit 1: lo; sq has at
+// least four k-blocks). Those rows hold no stream, their products are not stored, and wavefront w has
+// read them (another only in place of a k-block past the last, unused). One barrier inside; the
+// caller's next one frees them.
+__device__ __forceinline__ void rows_sums(const uint8_t *pw, int KB, uint8_t *sq, gemv::v4i &hi, gemv::v4i &lo) {
+    static_assert(MS_MAX == 8 && TDT_ROWS == 16, "lanes 0..31 hold the streams' sums, 16 bytes in each of the other rows");
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     hi = gemv::v4i{0, 0, 0, 0};
     lo = gemv::v4i{0, 0, 0, 0};
@@ -1557,16 +1560,17 @@ __device__ __forceinline__ void rows_sums(const uint8_t *pw, int KB, const uint8
             lo = __builtin_amdgcn_mfma_i32_16x16x64_i8(al[u], wv[u], lo, 0, 0, 0);
         }
     }
+    uint8_t *part = sq + (lane >> 3) * 256 + MS_MAX * 16 + (lane & 7) * 16;
     if (wave && lane < 4 * MS_MAX) {  // rows 4 (lane / 16) + 0..3: the streams'
-        sh.part[wave - 1][0][lane] = hi;
-        sh.part[wave - 1][1][lane] = lo;
+        *reinterpret_cast<gemv::v4i *>(part + wave * 2048) = hi;
+        *reinterpret_cast<gemv::v4i *>(part + wave * 2048 + 1024) = lo;
     }
     __syncthreads();
     if (wave == 0 && lane < 4 * MS_MAX) {
 #pragma unroll
-        for (int w = 0; w < RES_WAVES - 1; w++) {
-            hi += sh.part[w][0][lane];
-            lo += sh.part[w][1][lane];
+        for (int w = 1; w < RES_WAVES; w++) {
+            hi += *reinterpret_cast<const gemv::v4i *>(part + w * 2048);
+            lo += *reinterpret_cast<const gemv::v4i *>(part + w * 2048 + 1024);
         }
     }
 }
@@ -1989,7 +1993,7 @@ __global__ __launch_bounds__(RES_THREADS) void tdt_multi_kernel(MultiArgs a) {
             }
             for (int pi = 0; pi < npl; pi++) {
                 gemv::v4i hi, lo;
-                rows_sums(wlay + (size_t)pi * KBL * 1024, KBL, sq, sh, hi, lo);
+                rows_sums(wlay + (size_t)pi * KBL * 1024, KBL, sq, hi, lo);
                 if (wave == 0) {
                     const int j16 = lane & 15, orow = (lane >> 4) * 4, k = j16 & 3;
                     const float sc = sh.ls[l][pi * PANEL + j16], bs = sh.lbias[l][pi * PANEL + j16];
@@ -2035,7 +2039,7 @@ __global__ __launch_bounds__(RES_THREADS) void tdt_multi_kernel(MultiArgs a) {
             if (sh.abort) break;
             for (int pi = 0; pi < npp; pi++) {
                 gemv::v4i hi, lo;
-                rows_sums(wp + (size_t)pi * KBP * 1024, KBP, sq, sh, hi, lo);
+                rows_sums(wp + (size_t)pi * KBP * 1024, KBP, sq, hi, lo);
                 if (wave == 0) {
                     const int j16 = lane & 15, orow = (lane >> 4) * 4, col = (pp0 + pi) * PANEL + j16;
                     const float sc = sh.ps[pi * PANEL + j16], bs = sh.pbias[pi * PANEL + j16];

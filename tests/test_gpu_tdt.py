@@ -424,6 +424,10 @@ MULTI_EDGES = [  # h, vocab, layers, frames per stream
     (772, 90, 2, [12, 7, 10, 9, 11, 8, 13]),
     (36, 50, 4, [40, 1]),
     (192, 60, 2, [25, 19, 22, 30, 8, 27]),
+    # LDS near its end: the projection's panels beside the others' (no room for workgroups of their own),
+    # and in their place, two joint panels per workgroup.
+    (532, 30000, 1, [9, 6, 11, 8, 7, 10, 5, 12]),
+    (772, 4200, 2, [8, 12, 10, 7, 9]),
 ]
 
 
