@@ -694,23 +694,6 @@ __device__ __forceinline__ bool wait_words(const uint64_t *const (&p)[N], uint32
     }
 }
 
-// wait_words for the words at base + off[i].
-template <int N>
-__device__ __forceinline__ bool wait_offsets(const uint64_t *base, const uint32_t (&off)[N], uint32_t need,
-                                             const uint32_t (&tag)[N], uint64_t (&w)[N], const int32_t *err,
-                                             uint64_t deadline) {
-    for (int round = 0; need; round++) {
-#pragma unroll
-        for (int i = 0; i < N; i++)
-            if (need >> i & 1) w[i] = word_load(base + off[i]);
-#pragma unroll
-        for (int i = 0; i < N; i++)
-            if ((need >> i & 1) && (uint32_t)(w[i] >> 32) == tag[i]) need &= ~(1u << i);
-        if (need && (round & 15) == 15 && ((uint64_t)wall_clock64() > deadline || load_i(err) != 0)) return false;
-    }
-    return true;
-}
-
 // Copies np panels from p0 on of a matrix into LDS, panel pi's k-block t at (pi KB + t) * 1024.
 __device__ __forceinline__ void copy_panels(uint8_t *dst, const ResMat &m, int p0, int np) {
     const int per = m.KB * 64, total = np * per;
@@ -1469,43 +1452,91 @@ __device__ __forceinline__ void ms_fail(const MultiArgs &a, MultiShared &sh) {
     store_i(&a.ctl[0].err, 1);
 }
 
-// Waits for N chunks of four tagged words at words + off[i] (bit i of need), all loads issued before the
-// first wait: a round trip between workgroups costs about a microsecond. x[i] gets the values.
-template <int N>
-__device__ __forceinline__ bool wait_chunks(const uint64_t *words, const uint32_t (&off)[N], uint32_t need,
-                                            const uint32_t (&tag)[N], v4f (&x)[N], const int32_t *err, uint64_t ticks) {
-    uint64_t w[N][4];
+// Waits for rows of tagged words, all loads issued before the first wait: a round trip between workgroups
+// costs about a microsecond. Row rr (bit rr of need, rr < R) has CH chunks of four words at row[rr] and
+// carries tag[rr]; x[NC rr + i] gets chunk lane + 64 i (the last one past the row). Only x is per lane, so
+// addresses and tags stay in scalar registers: held per lane for every word, they spilled.
+template <int NC, int R>
+__device__ __forceinline__ bool wait_rows(const uint64_t *const (&row)[R], const uint32_t (&tag)[R], uint32_t need,
+                                          int CH, v4f (&x)[R * NC], const int32_t *err, uint64_t ticks) {
+    const int lane = threadIdx.x & 63;
+    uint64_t w[R * NC][4];
     const uint64_t deadline = (uint64_t)wall_clock64() + ticks;
     for (int round = 0; need; round++) {
 #pragma unroll
-        for (int i = 0; i < N; i++)
-            if (need >> i & 1) {
+        for (int rr = 0; rr < R; rr++)
+            if (need >> rr & 1) {
 #pragma unroll
-                for (int u = 0; u < 4; u++) w[i][u] = word_load(words + off[i] + u);
+                for (int i = 0; i < NC; i++)
+#pragma unroll
+                    for (int u = 0; u < 4; u++) w[NC * rr + i][u] = word_load(row[rr] + 4 * min(lane + 64 * i, CH - 1) + u);
             }
 #pragma unroll
-        for (int i = 0; i < N; i++)
-            if ((need >> i & 1) && (uint32_t)(w[i][0] >> 32) == tag[i] && (uint32_t)(w[i][1] >> 32) == tag[i] &&
-                (uint32_t)(w[i][2] >> 32) == tag[i] && (uint32_t)(w[i][3] >> 32) == tag[i]) {
-                x[i] = v4f{word_value(w[i][0]), word_value(w[i][1]), word_value(w[i][2]), word_value(w[i][3])};
-                need &= ~(1u << i);
+        for (int rr = 0; rr < R; rr++)
+            if (need >> rr & 1) {
+                bool here = true;
+#pragma unroll
+                for (int i = 0; i < NC; i++)
+#pragma unroll
+                    for (int u = 0; u < 4; u++) here = here && (uint32_t)(w[NC * rr + i][u] >> 32) == tag[rr];
+                if (__all(here)) {
+                    need &= ~(1u << rr);
+#pragma unroll
+                    for (int i = 0; i < NC; i++) {
+                        const uint64_t(&c)[4] = w[NC * rr + i];
+                        x[NC * rr + i] = v4f{word_value(c[0]), word_value(c[1]), word_value(c[2]), word_value(c[3])};
+                    }
+                }
             }
-        if (need && (round & 15) == 15 && ((uint64_t)wall_clock64() > deadline || load_i(err) != 0)) return false;
+        if (need && (round & 15) == 15 && __any((uint64_t)wall_clock64() > deadline || load_i(err) != 0)) return false;
     }
     return true;
 }
 
-// The exponents and digits of the wavefront's two streams' rows [first; second]: lane l holds chunks l +
-// 64 i of each half (CA and CB chunks, zero past them) (i < NC) of streams wave (xa[i]) and wave + 4 (xa[NC + i]), and
-// stream q is row q of the 16-row layout (k-block t, digit d at sq + t 2048 + d 1024, lane 16 g + q), zero
-// past the row up to KB k-blocks. Both rows in one stretch of code, so that their chains overlap.
+// Waits for the streams' predictions (stream q: bit q of need, words [2][M][h] at words, tag n[q]) and leaves
+// thread t's words t, t + 256, ... (NC of them, the last one past the row) in pin [M][h]; all loads at once.
 template <int NC>
-__device__ __forceinline__ void stream_digits(const v4f (&xa)[2 * NC], int CA, const v4f (&xb)[2 * NC], int CB, int KB,
-                                              uint8_t *sq, MultiShared &sh) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    int32_t e[2];
+__device__ __forceinline__ bool wait_preds(const uint64_t *words, int M, int h, const uint32_t (&n)[MS_MAX], uint32_t need,
+                                           float *pin, const int32_t *err, uint64_t ticks) {
+    const int tid = threadIdx.x;
+    uint64_t w[MS_MAX][NC];
+    const uint64_t deadline = (uint64_t)wall_clock64() + ticks;
+    for (int round = 0; need; round++) {
 #pragma unroll
-    for (int rr = 0; rr < 2; rr++) {
+        for (int q = 0; q < MS_MAX; q++)
+            if (need >> q & 1) {
+                const uint64_t *row = words + (size_t)((n[q] & 1) * M + q) * h;
+#pragma unroll
+                for (int v = 0; v < NC; v++) w[q][v] = word_load(row + min(tid + RES_THREADS * v, h - 1));
+            }
+#pragma unroll
+        for (int q = 0; q < MS_MAX; q++)
+            if (need >> q & 1) {
+                bool here = true;
+#pragma unroll
+                for (int v = 0; v < NC; v++) here = here && (uint32_t)(w[q][v] >> 32) == n[q];
+                if (__all(here)) {
+                    need &= ~(1u << q);
+#pragma unroll
+                    for (int v = 0; v < NC; v++) pin[(size_t)q * h + min(tid + RES_THREADS * v, h - 1)] = word_value(w[q][v]);
+                }
+            }
+        if (need && (round & 15) == 15 && __any((uint64_t)wall_clock64() > deadline || load_i(err) != 0)) return false;
+    }
+    return true;
+}
+
+// The exponents and digits of the rows [first; second] of the wavefront's R streams wave + 4 rr: lane l
+// holds chunks l + 64 i (i < NC) of each half (CA and CB chunks, past them copies of one or zero) in xa[NC rr + i] and xb[..].
+// Stream q is row q of the 16-row layout (k-block t, digit d at sq + t 2048 + d 1024, lane 16 g + q), zero
+// past the row up to KB k-blocks. The rows in one stretch of code, so that their chains overlap.
+template <int NC, int R>
+__device__ __forceinline__ void stream_digits(const v4f (&xa)[R * NC], int CA, const v4f (&xb)[R * NC], int CB, int KB,
+                                              uint8_t *sq, MultiShared &sh) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int32_t e[R];
+#pragma unroll
+    for (int rr = 0; rr < R; rr++) {
         uint32_t mx = 0;
 #pragma unroll
         for (int i = 0; i < NC; i++) mx = max(mx, max(chunk_max(xa[NC * rr + i]), chunk_max(xb[NC * rr + i])));
@@ -1520,7 +1551,7 @@ __device__ __forceinline__ void stream_digits(const v4f (&xa)[2 * NC], int CA, c
         *reinterpret_cast<uint32_t *>(d + 1024) = lo;
     };
 #pragma unroll
-    for (int rr = 0; rr < 2; rr++) {
+    for (int rr = 0; rr < R; rr++) {
 #pragma unroll
         for (int i = 0; i < NC; i++) {
             const int c = lane + 64 * i;
@@ -1538,28 +1569,32 @@ __device__ __forceinline__ void stream_digits(const v4f (&xa)[2 * NC], int CA, c
 // kernel: wavefront w's go to the rows from MS_MAX on of k-block w (digit 0: hi, digit 1: lo; sq has at
 // least four k-blocks). Those rows hold no stream, their products are not stored, and wavefront w has
 // read them (another only in place of a k-block past the last, unused). One barrier inside; the
-// caller's next one frees them.
+// caller's next one frees them. Up to five k-blocks are wavefront 0's alone: their MFMAs take less than
+// the barrier.
 __device__ __forceinline__ void rows_sums(const uint8_t *pw, int KB, uint8_t *sq, gemv::v4i &hi, gemv::v4i &lo) {
     static_assert(MS_MAX == 8 && TDT_ROWS == 16, "lanes 0..31 hold the streams' sums, 16 bytes in each of the other rows");
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     hi = gemv::v4i{0, 0, 0, 0};
     lo = gemv::v4i{0, 0, 0, 0};
-    for (int t0 = wave; t0 < KB; t0 += 5 * RES_WAVES) {  // five k-blocks' operands before their MFMAs
+    const bool split = KB > 5;
+    const int step = split ? RES_WAVES : 1;
+    for (int t0 = split || wave == 0 ? wave : KB; t0 < KB; t0 += 5 * step) {  // five k-blocks' operands before their MFMAs
         gemv::v4i ah[5], al[5], wv[5];
 #pragma unroll
         for (int u = 0; u < 5; u++) {
-            const int t = min(t0 + u * RES_WAVES, KB - 1);
+            const int t = min(t0 + u * step, KB - 1);
             ah[u] = *reinterpret_cast<const gemv::v4i *>(sq + t * 2048 + lane * 16);
             al[u] = *reinterpret_cast<const gemv::v4i *>(sq + t * 2048 + 1024 + lane * 16);
             wv[u] = *reinterpret_cast<const gemv::v4i *>(pw + (size_t)t * 1024 + lane * 16);
         }
 #pragma unroll
         for (int u = 0; u < 5; u++) {
-            if (t0 + u * RES_WAVES >= KB) break;
+            if (t0 + u * step >= KB) break;
             hi = __builtin_amdgcn_mfma_i32_16x16x64_i8(ah[u], wv[u], hi, 0, 0, 0);
             lo = __builtin_amdgcn_mfma_i32_16x16x64_i8(al[u], wv[u], lo, 0, 0, 0);
         }
     }
+    if (!split) return;
     uint8_t *part = sq + (lane >> 3) * 256 + MS_MAX * 16 + (lane & 7) * 16;
     if (wave && lane < 4 * MS_MAX) {  // rows 4 (lane / 16) + 0..3: the streams'
         *reinterpret_cast<gemv::v4i *>(part + wave * 2048) = hi;
@@ -1575,12 +1610,13 @@ __device__ __forceinline__ void rows_sums(const uint8_t *pw, int KB, uint8_t *sq
     }
 }
 
-// L: the most LSTM layers (a.layers <= L); NC: the chunks of 4 inputs a lane holds of h (h <= 256 NC).
-template <int L, int NC>
+// L: the most LSTM layers (a.layers <= L); NC: the chunks of 4 inputs a lane holds of h (h <= 256 NC); R: the
+// streams of a wavefront (M <= 4 R), wave and wave + 4.
+template <int L, int NC, int R>
 __global__ __launch_bounds__(RES_THREADS) void tdt_multi_kernel(MultiArgs a) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     __shared__ MultiShared sh;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, b = blockIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), b = blockIdx.x;
     const size_t rc = (size_t)(b % RES_COPIES) * a.cs;
     const int M = a.M, S = a.slots, h = a.h, NJ = a.joint.n, KBJ = a.joint.KB, KBL = a.lstm[0].KB, KBP = a.proj.KB;
     const int KBJ4 = (KBJ + 3) & ~3;
@@ -1653,26 +1689,27 @@ __global__ __launch_bounds__(RES_THREADS) void tdt_multi_kernel(MultiArgs a) {
     // LSTM outputs of this wavefront's streams wave and wave + 4 (lane l: chunks l + 64 i), kept from
     // the layer above's input or read while the decision is waited for, and the prediction counts they
     // belong to: the recurrent halves then cost nothing when a token comes.
-    v4f hr[L][2 * NC];
-    uint32_t hv[L][2];
+    v4f hr[L][R * NC];
+    uint32_t hv[L][R];
 #pragma unroll
     for (int l = 0; l < L; l++) {
 #pragma unroll
-        for (int i = 0; i < 2 * NC; i++) hr[l][i] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-        hv[l][0] = hv[l][1] = TAG_NONE;
+        for (int i = 0; i < R * NC; i++) hr[l][i] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int rr = 0; rr < R; rr++) hv[l][rr] = TAG_NONE;
     }
     // The LSTM outputs of layer l under prediction count tag(q) of the streams q (of this wavefront's
-    // two) for which want(q) holds, into x.
-    auto read_h = [&](int l, auto want, auto tag_of, v4f (&x)[2 * NC]) -> bool {
-        uint32_t off[2 * NC], tag[2 * NC], need = 0;
+    // R) for which want(q, its number of the R) holds, into x.
+    auto read_h = [&](int l, auto want, auto tag_of, v4f (&x)[R * NC]) -> bool {
+        const uint64_t *row[R];
+        uint32_t tag[R], need = 0;
 #pragma unroll
-        for (int i = 0; i < 2 * NC; i++) {
-            const int q = wave + RES_WAVES * (i / NC), qm = min(q, M - 1), c = lane + 64 * (i % NC);
-            tag[i] = tag_of(qm);
-            off[i] = (uint32_t)(((l * 2 + (int)(tag[i] & 1)) * M + qm) * h + 4 * min(c, CH - 1));
-            if (q < M && want(qm) && c < CH) need |= 1u << i;
+        for (int rr = 0; rr < R; rr++) {
+            const int q = wave + RES_WAVES * rr, qm = min(q, M - 1);
+            tag[rr] = __builtin_amdgcn_readfirstlane(tag_of(qm));
+            row[rr] = a.w_h + rc + (size_t)((l * 2 + (int)(tag[rr] & 1)) * M + qm) * h;
+            if (q < M && want(qm, rr)) need |= 1u << rr;
         }
-        return wait_chunks<2 * NC>(a.w_h + rc, off, need, tag, x, err, a.wait_ticks);
+        return wait_rows<NC, R>(row, tag, __builtin_amdgcn_readfirstlane(need), CH, x, err, a.wait_ticks);
     };
     __syncthreads();
 
@@ -1703,31 +1740,16 @@ __global__ __launch_bounds__(RES_THREADS) void tdt_multi_kernel(MultiArgs a) {
                 }
             }
             // The live streams' predictions (waited for only after they change), all of them at once.
-            uint32_t off[NC * MS_MAX], tag[NC * MS_MAX], need = 0;
-            uint64_t w[NC * MS_MAX];
-            bool fresh = false;
+            uint32_t nq[MS_MAX], fresh = 0;
 #pragma unroll
             for (int q = 0; q < MS_MAX; q++) {
                 const int qm = min(q, M - 1);
-                const uint32_t nq = sh.n[qm];
-                const bool wanted = q < M && !sh.st[qm][4] && sh.pin_n[qm] != nq;
-                fresh = fresh || wanted;  // uniform
-#pragma unroll
-                for (int v = 0; v < NC; v++) {
-                    const int i = tid + RES_THREADS * v;
-                    off[NC * q + v] = ((nq & 1) * M + qm) * h + min(i, h - 1);
-                    tag[NC * q + v] = nq;
-                    if (wanted && i < h) need |= 1u << (NC * q + v);
-                }
+                nq[q] = __builtin_amdgcn_readfirstlane(sh.n[qm]);
+                if (q < M && !sh.st[qm][4] && sh.pin_n[qm] != nq[q]) fresh |= 1u << q;
             }
+            fresh = __builtin_amdgcn_readfirstlane(fresh);
             if (fresh) {
-                if (!wait_offsets<NC * MS_MAX>(a.w_pred + rc, off, need, tag, w, err, (uint64_t)wall_clock64() + a.wait_ticks))
-                    ms_fail(a, sh);
-#pragma unroll
-                for (int q = 0; q < MS_MAX; q++)
-#pragma unroll
-                    for (int v = 0; v < NC; v++)
-                        if (need >> (NC * q + v) & 1) pin[(size_t)q * h + tid + RES_THREADS * v] = word_value(w[NC * q + v]);
+                if (!wait_preds<NC>(a.w_pred + rc, M, h, nq, fresh, pin, err, a.wait_ticks)) ms_fail(a, sh);
                 __syncthreads();
                 if (sh.abort) break;
                 if (tid < M) sh.pin_n[tid] = sh.n[tid];  // read again only after the barriers below
@@ -1840,10 +1862,10 @@ __global__ __launch_bounds__(RES_THREADS) void tdt_multi_kernel(MultiArgs a) {
 #pragma unroll
             for (int l = 0; l < L; l++) {
                 if (l >= a.layers) break;
-                auto want = [&](int q) { return !sh.st[q][4] && hv[l][q / RES_WAVES] != sh.n[q]; };
+                auto want = [&](int q, int rr) { return !sh.st[q][4] && hv[l][rr] != sh.n[q]; };
                 ok = read_h(l, want, [&](int q) { return sh.n[q]; }, hr[l]) && ok;
 #pragma unroll
-                for (int rr = 0; rr < 2; rr++) hv[l][rr] = sh.n[min(wave + RES_WAVES * rr, M - 1)];
+                for (int rr = 0; rr < R; rr++) hv[l][rr] = sh.n[min(wave + RES_WAVES * rr, M - 1)];
             }
             if (!ok) ms_fail(a, sh);
         }
@@ -1958,6 +1980,7 @@ __global__ __launch_bounds__(RES_THREADS) void tdt_multi_kernel(MultiArgs a) {
         // ---- The prediction network for the emitting streams, stream q as row q (the other rows hold
         // whatever digits were there and are not stored).
         auto emits = [&](int q) { return sh.dec[q][3] >= 0; };
+        auto emits_rr = [&](int q, int) { return emits(q); };
         auto next_tag = [&](int q) { return sh.n[q] + 1; };
         bool stop = false;
 #pragma unroll
@@ -1968,22 +1991,22 @@ __global__ __launch_bounds__(RES_THREADS) void tdt_multi_kernel(MultiArgs a) {
             // [the embedding row or the layer below's new outputs; this layer's old outputs].
             bool ok = true;
             if (l == 0) {
-                v4f x[2 * NC];
+                v4f x[R * NC];
 #pragma unroll
-                for (int i = 0; i < 2 * NC; i++) {
+                for (int i = 0; i < R * NC; i++) {
                     const int q = min(wave + RES_WAVES * (i / NC), M - 1), c = lane + 64 * (i % NC), tok = sh.dec[q][3];
                     x[i] = *reinterpret_cast<const v4f *>(c < CH && tok >= 0 ? a.emb + (size_t)tok * h + 4 * c
                                                                              : gemv::ZERO_CHUNK);
                 }
-                stream_digits<NC>(x, CH, hr[0], CH, KBL, sq, sh);
+                stream_digits<NC, R>(x, CH, hr[0], CH, KBL, sq, sh);
             } else {
-                ok = read_h(l - 1, emits, next_tag, hr[l > 0 ? l - 1 : 0]);
+                ok = read_h(l - 1, emits_rr, next_tag, hr[l > 0 ? l - 1 : 0]);
 #pragma unroll
-                for (int rr = 0; rr < 2; rr++) {
+                for (int rr = 0; rr < R; rr++) {
                     const int q = min(wave + RES_WAVES * rr, M - 1);
                     hv[l > 0 ? l - 1 : 0][rr] = sh.n[q] + (emits(q) ? 1 : 0);
                 }
-                stream_digits<NC>(hr[l > 0 ? l - 1 : 0], CH, hr[l], CH, KBL, sq, sh);
+                stream_digits<NC, R>(hr[l > 0 ? l - 1 : 0], CH, hr[l], CH, KBL, sq, sh);
             }
             if (!ok) ms_fail(a, sh);
             __syncthreads();
@@ -2030,11 +2053,11 @@ __global__ __launch_bounds__(RES_THREADS) void tdt_multi_kernel(MultiArgs a) {
         }
         if (stop) break;
         if (npp > 0) {
-            v4f x[2 * NC], none[2 * NC];
+            v4f x[R * NC], none[R * NC];
 #pragma unroll
-            for (int i = 0; i < 2 * NC; i++) x[i] = none[i] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-            if (!read_h(a.layers - 1, emits, next_tag, x)) ms_fail(a, sh);
-            stream_digits<NC>(x, CH, none, 0, KBP, sq, sh);
+            for (int i = 0; i < R * NC; i++) x[i] = none[i] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+            if (!read_h(a.layers - 1, emits_rr, next_tag, x)) ms_fail(a, sh);
+            stream_digits<NC, R>(x, CH, none, 0, KBP, sq, sh);
             __syncthreads();
             if (sh.abort) break;
             for (int pi = 0; pi < npp; pi++) {
@@ -2332,10 +2355,19 @@ static size_t multi_lds(const TdtNet &net, const TdtPlan &p) {
            (M * net.h + 2 * net.layers * M * p.LP * 4 + M * p.PP * PANEL) * sizeof(float);
 }
 
-static const void *multi_kernel(const TdtNet &net) {
-    static_assert(TDT_MAX_H <= 4 * 256, "four chunks per lane");
-    return net.layers <= 2 && net.h <= 3 * 256 ? reinterpret_cast<const void *>(&tdt_multi_kernel<2, 3>)
-                                               : reinterpret_cast<const void *>(&tdt_multi_kernel<TDT_MAX_LAYERS, 4>);
+// The instance for m streams. What a lane holds of its streams' rows is in registers, so the fewer layers,
+// chunks and streams an instance has room for, the shorter its code and its chains; the widest one alone
+// spilled and lost to one row at a time. us, 375 frames: 4 layers of 320 units, 2 streams 7790 with
+// <4, 4, 2> for all beyond two layers or 768 units, 6550 one row at a time, 5970 with R = 1; 4 layers of 64 units,
+// 2 streams 10830, 7640 and 8085, and 6210 with NC = 1 (2 layers 5870, 5120, 5150 and 4250).
+static const void *multi_kernel(const TdtNet &net, size_t m) {
+    static_assert(TDT_MAX_H <= 4 * 256 && TDT_MAX_STREAMS <= 2 * RES_WAVES, "four chunks per lane, two streams per wavefront");
+    auto of = [m](auto one, auto two) {
+        return m > (size_t)RES_WAVES ? reinterpret_cast<const void *>(two) : reinterpret_cast<const void *>(one);
+    };
+    if (net.h <= 256) return of(&tdt_multi_kernel<TDT_MAX_LAYERS, 1, 1>, &tdt_multi_kernel<TDT_MAX_LAYERS, 1, 2>);
+    if (net.layers <= 2 && net.h <= 3 * 256) return of(&tdt_multi_kernel<2, 3, 1>, &tdt_multi_kernel<2, 3, 2>);
+    return of(&tdt_multi_kernel<TDT_MAX_LAYERS, 4, 1>, &tdt_multi_kernel<TDT_MAX_LAYERS, 4, 2>);
 }
 
 bool tdt_multi_plan(const TdtNet &net, TdtPlan &plan) {
@@ -2347,14 +2379,16 @@ bool tdt_multi_plan(const TdtNet &net, TdtPlan &plan) {
         hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess)
         return false;
     const size_t lds = multi_lds(net, plan);
-    const void *f = multi_kernel(net);
-    hipFuncAttributes fa;
-    if (hipFuncGetAttributes(&fa, f) != hipSuccess || lds + fa.sharedSizeBytes > (size_t)max_lds) return false;
-    if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) return false;
-    int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, f, RES_THREADS, lds) != hipSuccess || per_cu < 1 ||
-        (size_t)plan.grid > (size_t)per_cu * cus)
-        return false;
+    for (size_t m : {(size_t)RES_WAVES, TDT_MAX_STREAMS}) {
+        const void *f = multi_kernel(net, m);
+        hipFuncAttributes fa;
+        if (hipFuncGetAttributes(&fa, f) != hipSuccess || lds + fa.sharedSizeBytes > (size_t)max_lds) return false;
+        if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) return false;
+        int per_cu = 0;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, f, RES_THREADS, lds) != hipSuccess || per_cu < 1 ||
+            (size_t)plan.grid > (size_t)per_cu * cus)
+            return false;
+    }
     plan.mlds = lds;
     plan.multi = true;
     return true;
@@ -2422,7 +2456,7 @@ hipError_t launch_tdt_multi(TdtCtl *ctl, const TdtNet &net, const TdtPlan &plan,
     a.steps = steps;
     a.wait_ticks = wait_ticks;
     void *args[] = {&a};
-    return hipLaunchCooperativeKernel(multi_kernel(net), dim3((unsigned)plan.grid), dim3(RES_THREADS), args,
+    return hipLaunchCooperativeKernel(multi_kernel(net, m), dim3((unsigned)plan.grid), dim3(RES_THREADS), args,
                                       (unsigned)plan.mlds, s);
 }
 

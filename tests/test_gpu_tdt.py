@@ -416,14 +416,20 @@ def test_multi_stream_decode_matches_each_stream(tk, orc, case):
     dec.close()
 
 
-# The multi-stream kernel's instances (up to two layers of at most 768 units, else), rows that end inside
-# a k-block, one to eight streams over the four wavefronts.
+# The multi-stream kernel's instances (at most 256 units; up to two layers of at most 768; else; each for up
+# to four streams and for more), products of up to five k-blocks and of more, rows that end inside a
+# k-block, one to eight streams over the four wavefronts.
 MULTI_EDGES = [  # h, vocab, layers, frames per stream
     (100, 70, 3, [20, 31, 5, 18, 26]),
     (768, 90, 2, [9, 14, 11]),
     (772, 90, 2, [12, 7, 10, 9, 11, 8, 13]),
     (36, 50, 4, [40, 1]),
     (192, 60, 2, [25, 19, 22, 30, 8, 27]),
+    (160, 60, 2, [14, 22, 9]),
+    (164, 60, 1, [14, 22, 9, 17]),
+    (256, 80, 4, [11, 8, 15, 9, 12, 7, 10, 13]),
+    (260, 80, 3, [10, 13, 6, 12]),
+    (960, 70, 1, [9, 12, 8]),
     # LDS near its end: the projection's panels beside the others' (no room for workgroups of their own),
     # and in their place, two joint panels per workgroup.
     (532, 30000, 1, [9, 6, 11, 8, 7, 10, 5, 12]),
@@ -434,7 +440,8 @@ MULTI_EDGES = [  # h, vocab, layers, frames per stream
 @pytest.mark.parametrize("h,vocab,layers,frames", MULTI_EDGES)
 def test_multi_stream_decode_at_its_edges_is_each_stream_alone(tk, h, vocab, layers, frames):
     """Tokens, position, state and prediction of every stream, bit for bit those of the single-stream
-    decode (which the other tests hold against the oracle), twice over from the states of the first."""
+    decode (which the other tests hold against the oracle), twice over from the states of the first, the
+    second time in launches of three steps."""
     import torch
 
     rng = np.random.default_rng(7 * h + layers)
@@ -445,10 +452,12 @@ def test_multi_stream_decode_at_its_edges_is_each_stream_alone(tk, h, vocab, lay
     pd = [dev((0.3 * rng.standard_normal(h)).astype(np.float32)) for _ in frames]
     s1, p1 = [t.clone() for t in sd], [t.clone() for t in pd]
     for turn in range(2):
+        dec.set_resident_limits(steps_per_launch=3 * turn)
         encs = [dev(rng.standard_normal((f, h)).astype(np.float32)) for f in frames]
         say("multi-stream edges", h, vocab, layers, frames, turn)
         got = dec.decode_streams(encs, sd, pd)
         assert dec.last_resident == 2
+        dec.set_resident_limits()
         for q, enc in enumerate(encs):
             assert dec.decode(enc, s1[q], p1[q]) == got[q], q
             assert torch.equal(sd[q].view(torch.int32), s1[q].view(torch.int32)), q
