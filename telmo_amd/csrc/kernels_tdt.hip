@@ -132,7 +132,8 @@ __device__ __forceinline__ float quad_lane(float v) {
 // lanes of a quad hold one unit's gates of the same four rows; lane k of it applies the cell update
 // (src/parakeet.rs:1549-1562) to row k: c = f c + i g, h = o tanh(c), each product rounded before the
 // sum. The old cells are requested before the products: with one lane updating the four rows in turn,
-// each read waiting behind the row before's stores, a layer of eight rows took 10.5 us.
+// each read waiting behind the row before's stores, a layer of eight rows took 10.5 us. One row (the
+// decode's) is lane 0's of the quad alone.
 struct LstmOut {
     static constexpr bool ROWS4 = true;
     const float *s_in;
@@ -152,6 +153,7 @@ struct LstmOut {
         float gate[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int r = 0; r < 4; r++) {
+            if (r > 0 && m == 1) break;
             const float g[4] = {quad_lane<0>(v[r]), quad_lane<1>(v[r]), quad_lane<2>(v[r]), quad_lane<3>(v[r])};
 #pragma unroll
             for (int q = 0; q < 4; q++) gate[q] = k == r ? g[q] : gate[q];
