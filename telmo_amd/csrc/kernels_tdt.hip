@@ -1023,7 +1023,7 @@ __global__ __launch_bounds__(RES_THREADS) void tdt_resident_kernel(ResArgs a) {
             // Wavefront w scores panels w, w + 4, ... of this workgroup, the weights as the first operand:
             // element v of lane l is row l % 16, column 4 (l / 16) + v, so a row's best entries meet over
             // a lane's four columns and then four lanes (with the rows first, over sixteen lanes for
-            // each of a lane's four rows: 60 s decoded 5940 us, so 5693). Each row keeps its best vocabulary entry and its best
+            // each of a lane's four rows: 60 s decoded 6960 us, so 6636). Each row keeps its best vocabulary entry and its best
             // duration entry (index d for column vocab + d). A NaN first logit (column 0) is never
             // beaten in the reference's argmax: it enters as (+inf, 0), which nothing comes before;
             // a NaN first duration logit likewise.
@@ -1035,18 +1035,21 @@ __global__ __launch_bounds__(RES_THREADS) void tdt_resident_kernel(ResArgs a) {
                 if constexpr (Q8) {
                     // Half hh of k-block t is block 2 t + hh: lane 16 g + x reads 8 bytes of layout
                     // lane 16 (2 hh + g / 2) + x, the same inputs for the digits and the weights. Both
-                    // halves' MFMAs are issued before their folds, which run in block order.
+                    // halves' MFMAs are issued before their folds, which run in block order, and their scales
+                    // (four columns' here) are read before the MFMAs: after them, 60 s took 1% longer.
                     const uint8_t *wb = wj + (size_t)pi * KBJ * 1024;
                     const float *ds = qsj + (size_t)pi * NBJ * PANEL + c4;
                     const int g = lane >> 4, off0 = (16 * (g >> 1) + j16) * 16 + 8 * (g & 1);
                     for (int t = 0; t < KBJ; t++) {
                         gemv::v4i H[2], L[2];
+                        v4f d[2];
 #pragma unroll
                         for (int hh = 0; hh < 2; hh++) {
                             const int off = off0 + hh * 512;
                             const long ah = *reinterpret_cast<const long *>(sq + t * 2048 + off);
                             const long al = *reinterpret_cast<const long *>(sq + t * 2048 + 1024 + off);
                             const long wv = *reinterpret_cast<const long *>(wb + (size_t)t * 1024 + off);
+                            d[hh] = *reinterpret_cast<const v4f *>(ds + min(2 * t + hh, NBJ - 1) * PANEL);
                             H[hh] = __builtin_amdgcn_mfma_i32_16x16x32_i8(wv, ah, gemv::v4i{0, 0, 0, 0}, 0, 0, 0);
                             L[hh] = __builtin_amdgcn_mfma_i32_16x16x32_i8(wv, al, gemv::v4i{0, 0, 0, 0}, 0, 0, 0);
                         }
@@ -1054,9 +1057,8 @@ __global__ __launch_bounds__(RES_THREADS) void tdt_resident_kernel(ResArgs a) {
                         for (int hh = 0; hh < 2; hh++) {
                             const int bk = 2 * t + hh;
                             if (bk < NBJ) {
-                                const v4f d = *reinterpret_cast<const v4f *>(ds + bk * PANEL);
 #pragma unroll
-                                for (int v = 0; v < 4; v++) fq[v] = __builtin_fmaf(d[v], (float)(H[hh][v] * 256 + L[hh][v]), fq[v]);
+                                for (int v = 0; v < 4; v++) fq[v] = __builtin_fmaf(d[hh][v], (float)(H[hh][v] * 256 + L[hh][v]), fq[v]);
                             }
                         }
                     }

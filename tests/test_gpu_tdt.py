@@ -65,6 +65,7 @@ DECODE_CASES = [  # h, vocab, durations, layers, precision, frames, blank_bias, 
     (64, 100, [0, 1, 2, 3, 4], 2, INT8_P, 200, 6.0, 3),
     (128, 300, [0, 2, 4], 1, INT8_P, 77, 4.0, 2),
     (64, 100, [1, 2], 3, Q8_0_P, 50, 2.0, 5),
+    (96, 70, [0, 1, 2], 2, Q8_0_P, 40, 3.0, 4),  # an odd number of 32-input blocks
     (640, 8193, [0, 1, 2, 3, 4], 2, INT8_P, 120, 6.0, 10),
     (640, 8193, [0, 1, 2, 3, 4], 2, Q8_0_P, 60, 6.0, 10),
 ]
