@@ -166,6 +166,39 @@ struct ExactArgs {
     int vec;     // outputs are 16-byte aligned and rows hold whole runs of four
 };
 
+// The epilogue and stores of RB blocks of 16 rows from m0 on and one panel: lane (lg, lj) holds columns
+// 4 lg + 0..3 of row lj of each block.
+template <int RB>
+__device__ __forceinline__ void store_blocks(const ExactArgs &g, const v4f (&acc)[RB], int m0, int panel) {
+    const int lane = threadIdx.x & 63, lg = lane >> 4, lj = lane & 15;
+    const bool has_bias = g.epi.bias != nullptr, accumulate = g.epi.accumulate != 0;
+    const int col = panel * PANEL + 4 * lg;
+    if (col >= g.N) return;
+    float bias[4];
+#pragma unroll
+    for (int v = 0; v < 4; v++) bias[v] = has_bias && col + v < g.N ? g.epi.bias[col + v] : 0.0f;
+#pragma unroll
+    for (int r = 0; r < RB; r++) {
+        const int row = m0 + r * 16 + lj;
+        if (row >= g.M) continue;
+        float *cp = g.c + (size_t)row * g.ldc + col;
+        if (g.vec) {
+            v4f old = {0.0f, 0.0f, 0.0f, 0.0f}, y;
+            if (accumulate) old = *reinterpret_cast<const v4f *>(cp);
+#pragma unroll
+            for (int v = 0; v < 4; v++)
+                y[v] = epilogue_vals(acc[r][v], has_bias, bias[v], g.epi.act, g.epi.scale, accumulate, old[v]);
+            *reinterpret_cast<v4f *>(cp) = y;
+        } else {
+#pragma unroll
+            for (int v = 0; v < 4; v++)
+                if (col + v < g.N)
+                    cp[v] = epilogue_vals(acc[r][v], has_bias, bias[v], g.epi.act, g.epi.scale, accumulate,
+                                          accumulate ? cp[v] : 0.0f);
+        }
+    }
+}
+
 // PREC: the right-hand side's precision. AW, BW: A rows / the f32 right-hand side take 16-byte copies.
 template <uint32_t PREC, int RB, int NS, bool AW, bool BW>
 __global__ __launch_bounds__(EXACT_THREADS) void exact_kernel(ExactArgs g) {
@@ -406,33 +439,53 @@ __global__ __launch_bounds__(EXACT_THREADS) void exact_kernel(ExactArgs g) {
         else mma_ragged(f1, left - 32);
     }
 
-    // Lane (lg, lj) holds columns 4 lg + 0..3 of row lj of each block.
-    const bool has_bias = g.epi.bias != nullptr, accumulate = g.epi.accumulate != 0;
-    const int col = panel * PANEL + 4 * lg;
-    if (col >= g.N) return;
-    float bias[4];
+    store_blocks<RB>(g, acc, m0, panel);
+}
+
+// Sums of few inputs, without the ring: a wavefront takes 16 RB rows of one panel and loads its operands
+// in the MFMAs' layout straight from memory, four steps at a time, so no workgroup holds LDS or waits at a
+// barrier. Such products are bound by their stores and by how many workgroups are under way, and with the
+// ring's LDS one or two fit on a CU. us, 100,000 rows by 64 outputs with the ring / here, f32: 1 input
+// 46.5 / 10.1, 16 inputs 48.3 / 19.9, 32 inputs 50.6 / 31.8; f16: 1 input 21.2 / 10.5, 16 inputs 22.3 / 19.6, 24
+// inputs 22.9 / 26.8. 10,000 rows by 1024: f32, 32 inputs 48.6 / 43.9, 48 inputs 52.4 / 60.1; int8, 16 inputs
+// 28.1 / 27.5, 24 inputs 29.8 / 38.0. Hence the most inputs that it takes; the ring's four wavefronts
+// share the rows, which longer sums read often.
+template <uint32_t PREC>
+constexpr int SHORT = PREC == F32 ? 32 : 16;
+template <uint32_t PREC, int RB>
+__global__ __launch_bounds__(EXACT_THREADS) void exact_short_kernel(ExactArgs g) {
+    const int lane = threadIdx.x & 63, lg = lane >> 4, lj = lane & 15;
+    const int tile = blockIdx.x * (EXACT_THREADS / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int panel = tile % g.P, m0 = tile / g.P * RB * 16;
+    if (m0 >= g.M) return;
+    const float *row[RB];
 #pragma unroll
-    for (int v = 0; v < 4; v++) bias[v] = has_bias && col + v < g.N ? g.epi.bias[col + v] : 0.0f;
+    for (int r = 0; r < RB; r++) row[r] = g.a + (size_t)min(m0 + r * 16 + lj, g.M - 1) * g.lda;
+    v4f acc[RB];
 #pragma unroll
-    for (int r = 0; r < RB; r++) {
-        const int row = m0 + r * 16 + lj;
-        if (row >= g.M) continue;
-        float *cp = g.c + (size_t)row * g.ldc + col;
-        if (g.vec) {
-            v4f old = {0.0f, 0.0f, 0.0f, 0.0f}, y;
-            if (accumulate) old = *reinterpret_cast<const v4f *>(cp);
+    for (int r = 0; r < RB; r++) acc[r] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int i0 = 0; i0 < g.K; i0 += 16) {
+        float w[4], a[RB][4];
 #pragma unroll
-            for (int v = 0; v < 4; v++)
-                y[v] = epilogue_vals(acc[r][v], has_bias, bias[v], g.epi.act, g.epi.scale, accumulate, old[v]);
-            *reinterpret_cast<v4f *>(cp) = y;
-        } else {
+        for (int s = 0; s < 4; s++) {
+            const int i = i0 + 4 * s + lg, in = min(i, g.K - 1);
+            float v;
+            if constexpr (PREC == F32)
+                v = reinterpret_cast<const float *>(g.b)[(size_t)panel * g.pstride + (size_t)in * g.istride + lj];
+            else
+                v = widen_one(g.b, g.scales, PREC, g.K, g.pstride, g.istride, panel, lj, in);
+            w[s] = i < g.K ? v : 0.0f;
 #pragma unroll
-            for (int v = 0; v < 4; v++)
-                if (col + v < g.N)
-                    cp[v] = epilogue_vals(acc[r][v], has_bias, bias[v], g.epi.act, g.epi.scale, accumulate,
-                                          accumulate ? cp[v] : 0.0f);
+            for (int r = 0; r < RB; r++) a[r][s] = i < g.K ? row[r][in] : -0.0f;
+        }
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+            if (i0 + 4 * s >= g.K) break;
+#pragma unroll
+            for (int r = 0; r < RB; r++) acc[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[s], a[r][s], acc[r], 0, 0, 0);
         }
     }
+    store_blocks<RB>(g, acc, m0, panel);
 }
 
 template <uint32_t PREC, int RB, int NS>
@@ -448,12 +501,23 @@ hipError_t launch_tiles(ExactArgs g, bool aw, bool bw, hipStream_t s) {
     return hipGetLastError();
 }
 
+template <uint32_t PREC, int RB>
+hipError_t launch_short(const ExactArgs &g, hipStream_t s) {
+    const size_t tiles = (size_t)g.P * div_ceil((size_t)g.M, (size_t)(RB * 16));
+    const size_t groups = div_ceil(tiles, (size_t)(EXACT_THREADS / 64));
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(exact_short_kernel<PREC, RB>), dim3((unsigned)groups), dim3(EXACT_THREADS), 0, s, g);
+    return hipGetLastError();
+}
+
 template <uint32_t PREC>
 hipError_t launch_exact_as(ExactArgs g, hipStream_t s) {
     // 16-byte copies of rows that are 16 bytes aligned; their lane offsets are 32-bit over 64 rows.
     const bool aw = reinterpret_cast<uintptr_t>(g.a) % 16 == 0 && g.lda % 4 == 0 && g.lda < ((size_t)1 << 24);
     const bool bw = reinterpret_cast<uintptr_t>(g.b) % 16 == 0 && g.istride % 4 == 0 && g.istride < ((size_t)1 << 24);
     g.vec = ((reinterpret_cast<uintptr_t>(g.c) | g.ldc * sizeof(float)) % 16) == 0 && g.N % 4 == 0;
+    // Few inputs: four row blocks per wavefront where that leaves four wavefronts per CU.
+    if (g.K <= SHORT<PREC>)
+        return (size_t)g.P * g.M >= (size_t)64 * GFX950_CUS * 16 ? launch_short<PREC, 4>(g, s) : launch_short<PREC, 1>(g, s);
     // Row blocks per workgroup: the fewest row blocks on the busiest CU (workgroups per CU, rounded up,
     // times RB), and of equals the largest, whose widenings serve more MFMAs. us, f16, RB = 1 / 2 / 3 /
     // 4: 93 x 4096 -> 1024 24.2 / 39.6 / 53.5 / 69.2; 375 x 4096 -> 1024 43.6 / 42.6 / 56.7 / 71.4;

@@ -66,8 +66,10 @@ def test_exact_mode_is_bit_identical_to_the_fused_reference(tk, orc, p):
 
 # Row blocks per workgroup 1 to 4 (375, 750 and 1000 rows by 1024 outputs take 2, 3 and 4), ragged rows,
 # outputs and inputs (64 inputs per stage; one more, one less, several stages of the ring and a bit).
+# Then the kernel of short sums (up to 16 inputs, 32 of f32 values): one row block and four (66,000 rows).
 EXACT_TILES = [(1, 64, 16), (17, 65, 40), (33, 63, 33), (93, 448, 70), (375, 193, 1021), (750, 257, 1024),
-               (745, 96, 1010), (1000, 128, 1024), (990, 321, 1020)]
+               (745, 96, 1010), (1000, 128, 1024), (990, 321, 1020),
+               (1, 1, 1), (17, 3, 15), (33, 16, 33), (100, 4, 70), (31, 31, 20), (40, 32, 48), (45, 17, 16), (66000, 5, 70)]
 
 
 @pytest.mark.parametrize("m,k,n", EXACT_TILES)
@@ -104,7 +106,7 @@ def test_exact_products_on_each_tile_are_the_fused_reference(tk, orc, p, m, k, n
         w.close()
 
 
-@pytest.mark.parametrize("k", [31, 64, 65, 200])
+@pytest.mark.parametrize("k", [5, 16, 31, 64, 65, 200])
 def test_exact_sums_keep_subnormals_signed_zeros_and_infinities(tk, orc, k):
     """Sums that underflow to -0, subnormal inputs and products, infinities and NaN: the fused
     reference's bits (any NaN for a NaN), whatever the padding of the last stage."""
@@ -690,7 +692,8 @@ def test_large_products_with_unaligned_rows_or_bias(tk, orc, m, k, n, ldc, bias_
     w.close()
 
 
-@pytest.mark.parametrize("m,k,n,ldb", [(7, 128, 255, 255), (40, 128, 255, 256), (1, 33, 16, 20), (130, 300, 40, 64)])
+@pytest.mark.parametrize("m,k,n,ldb", [(7, 128, 255, 255), (40, 128, 255, 256), (1, 33, 16, 20), (130, 300, 40, 64),
+                                       (50, 5, 33, 51), (18, 32, 70, 80)])
 def test_rowmajor_right_hand_side_is_the_fused_reference(tk, orc, m, k, n, ldb):
     """BView::row_major (f32 activations as the right-hand side) gives the fused reference's bits: the
     same values packed into panels through the oracle's fused matmul. The shapes include the
