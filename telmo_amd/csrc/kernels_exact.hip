@@ -488,25 +488,46 @@ __global__ __launch_bounds__(EXACT_THREADS) void exact_short_kernel(ExactArgs g)
     store_blocks<RB>(g, acc, m0, panel);
 }
 
+// launch(g) for runs of rows, whole blocks of `rows` of them: about RUN_GROUPS workgroups each, since HIP
+// refuses launches of 2^32 threads, which 2^30 rows by one panel would be. A run takes milliseconds.
+constexpr size_t RUN_GROUPS = (size_t)1 << 20;
+template <class F>
+hipError_t launch_runs(ExactArgs g, size_t groups_per_block, size_t rows, F launch) {
+    const float *a = g.a;
+    float *c = g.c;
+    const size_t m = (size_t)g.M, run = std::max<size_t>(1, RUN_GROUPS / groups_per_block) * rows;
+    for (size_t m0 = 0; m0 < m; m0 += run) {
+        g.a = a + m0 * g.lda;
+        g.c = c + m0 * g.ldc;
+        g.M = (int)std::min(run, m - m0);
+        launch(g);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+}
+
 template <uint32_t PREC, int RB, int NS>
 hipError_t launch_tiles(ExactArgs g, bool aw, bool bw, hipStream_t s) {
     g.grid_n = (int)div_ceil((size_t)g.P, (size_t)4);
-    const size_t tiles = (size_t)g.grid_n * div_ceil((size_t)g.M, (size_t)(RB * 16));
-    if (tiles > (size_t)INT32_MAX) return hipErrorInvalidValue;
     auto kernel = aw ? &exact_kernel<PREC, RB, NS, true, true> : &exact_kernel<PREC, RB, NS, false, true>;
     if constexpr (PREC == F32) {
         if (!bw) kernel = aw ? &exact_kernel<PREC, RB, NS, true, false> : &exact_kernel<PREC, RB, NS, false, false>;
     }
-    hipLaunchKernelGGL(kernel, dim3((unsigned)tiles), dim3(EXACT_THREADS), 0, s, g);
-    return hipGetLastError();
+    return launch_runs(g, (size_t)g.grid_n, RB * 16, [&](const ExactArgs &r) {
+        const size_t tiles = (size_t)r.grid_n * div_ceil((size_t)r.M, (size_t)(RB * 16));
+        hipLaunchKernelGGL(kernel, dim3((unsigned)tiles), dim3(EXACT_THREADS), 0, s, r);
+    });
 }
 
 template <uint32_t PREC, int RB>
 hipError_t launch_short(const ExactArgs &g, hipStream_t s) {
-    const size_t tiles = (size_t)g.P * div_ceil((size_t)g.M, (size_t)(RB * 16));
-    const size_t groups = div_ceil(tiles, (size_t)(EXACT_THREADS / 64));
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(exact_short_kernel<PREC, RB>), dim3((unsigned)groups), dim3(EXACT_THREADS), 0, s, g);
-    return hipGetLastError();
+    constexpr size_t WAVES = EXACT_THREADS / 64;
+    return launch_runs(g, div_ceil((size_t)g.P, WAVES), RB * 16, [&](const ExactArgs &r) {
+        const size_t tiles = (size_t)r.P * div_ceil((size_t)r.M, (size_t)(RB * 16));
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(exact_short_kernel<PREC, RB>), dim3((unsigned)div_ceil(tiles, WAVES)),
+                           dim3(EXACT_THREADS), 0, s, r);
+    });
 }
 
 template <uint32_t PREC>
@@ -515,7 +536,7 @@ hipError_t launch_exact_as(ExactArgs g, hipStream_t s) {
     const bool aw = reinterpret_cast<uintptr_t>(g.a) % 16 == 0 && g.lda % 4 == 0 && g.lda < ((size_t)1 << 24);
     const bool bw = reinterpret_cast<uintptr_t>(g.b) % 16 == 0 && g.istride % 4 == 0 && g.istride < ((size_t)1 << 24);
     g.vec = ((reinterpret_cast<uintptr_t>(g.c) | g.ldc * sizeof(float)) % 16) == 0 && g.N % 4 == 0;
-    // Few inputs: four row blocks per wavefront where that leaves four wavefronts per CU.
+    // Few inputs: four row blocks per wavefront where that leaves sixteen wavefronts per CU.
     if (g.K <= SHORT<PREC>)
         return (size_t)g.P * g.M >= (size_t)64 * GFX950_CUS * 16 ? launch_short<PREC, 4>(g, s) : launch_short<PREC, 1>(g, s);
     // Row blocks per workgroup: the fewest row blocks on the busiest CU (workgroups per CU, rounded up,

@@ -106,6 +106,37 @@ def test_exact_products_on_each_tile_are_the_fused_reference(tk, orc, p, m, k, n
         w.close()
 
 
+@pytest.mark.parametrize("m,k,n,p", [((1 << 30) + 70, 1, 1, F32), ((1 << 26) + 70, 17, 3, F16)])
+def test_exact_products_of_more_rows_than_one_launch_takes(tk, orc, m, k, n, p):
+    """More than 2^32 threads' worth of rows (short sums), and more than one run of the ring's tiles: the
+    fused reference's bits in rows around the runs' borders and the last ones, an accumulating output."""
+    import torch
+
+    import telmo_amd
+
+    if torch.cuda.mem_get_info()[0] < 24 << 30:
+        pytest.skip("needs 24 GiB of GPU memory")
+    values, scales = orc.encode(orc.random(n * k, 2), n, k, p)
+    w = telmo_amd.PackedWeights.from_parts(tk, n, k, telmo_amd.Precision(p), values, scales)
+    a = torch.rand((m, k), device="cuda")
+    c = torch.ones((m, n), device="cuda")
+    torch.cuda.synchronize()
+    tk.set_mode(tk.EXACT)
+    say("exact rows", m, k, n)
+    try:
+        tk.matmul_device(a, k, m, w, c, n, telmo_amd.Epilogue(scale=0.5, accumulate=True))
+        tk.synchronize()
+    finally:
+        tk.set_mode(tk.FAST)
+        w.close()
+    for at in [0] + [i << 26 for i in range(1, (m >> 26) + 1)] + [m]:
+        r0, r1 = max(at - 70, 0), min(at + 70, m)
+        want = np.ones((r1 - r0) * n, np.float32)
+        rows = a[r0:r1].cpu().numpy().reshape(-1)
+        assert orc.matmul(True, rows, k, r1 - r0, values, scales, p, n, k, want, n, None, NONE, 0.5, True) == 0
+        assert np.array_equal(c[r0:r1].cpu().numpy().reshape(-1).view(np.uint32), want.view(np.uint32)), at
+
+
 @pytest.mark.parametrize("k", [5, 16, 31, 64, 65, 200])
 def test_exact_sums_keep_subnormals_signed_zeros_and_infinities(tk, orc, k):
     """Sums that underflow to -0, subnormal inputs and products, infinities and NaN: the fused
