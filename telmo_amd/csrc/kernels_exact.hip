@@ -489,10 +489,12 @@ __global__ __launch_bounds__(EXACT_THREADS) void exact_short_kernel(ExactArgs g)
 }
 
 // launch(g) for runs of rows, whole blocks of `rows` of them: about RUN_GROUPS workgroups each, since HIP
-// refuses launches of 2^32 threads, which 2^30 rows by one panel would be. A run takes milliseconds.
+// cuts the number of threads to 32 bits without an error: 2^30 + 70 rows by one panel in one launch left
+// all but the first rows as they were. A run takes milliseconds.
 constexpr size_t RUN_GROUPS = (size_t)1 << 20;
 template <class F>
 hipError_t launch_runs(ExactArgs g, size_t groups_per_block, size_t rows, F launch) {
+    if (groups_per_block * EXACT_THREADS > (size_t)UINT32_MAX) return hipErrorInvalidValue;
     const float *a = g.a;
     float *c = g.c;
     const size_t m = (size_t)g.M, run = std::max<size_t>(1, RUN_GROUPS / groups_per_block) * rows;
