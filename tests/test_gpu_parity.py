@@ -65,10 +65,13 @@ def test_exact_mode_is_bit_identical_to_the_fused_reference(tk, orc, p):
 
 
 # Row blocks per workgroup 1 to 4 (375, 750 and 1000 rows by 1024 outputs take 2, 3 and 4), ragged rows,
-# outputs and inputs (64 inputs per stage; one more, one less, several stages of the ring and a bit).
+# outputs and inputs (64 inputs per stage; one more, one less, some stages and a bit). The loop over whole
+# rounds of the ring (four stages with one row block, three otherwise) runs twice, and then the ragged tail,
+# for (93, 769), (375, 577), (750, 577) and (1000, 577); once for (93, 448) and (990, 321); the others miss it.
 # Then the kernel of short sums (up to 16 inputs, 32 of f32 values): one row block and four (66,000 rows).
 EXACT_TILES = [(1, 64, 16), (17, 65, 40), (33, 63, 33), (93, 448, 70), (375, 193, 1021), (750, 257, 1024),
                (745, 96, 1010), (1000, 128, 1024), (990, 321, 1020),
+               (93, 769, 70), (375, 577, 1021), (750, 577, 1024), (1000, 577, 1024),
                (1, 1, 1), (17, 3, 15), (33, 16, 33), (100, 4, 70), (31, 31, 20), (40, 32, 48), (45, 17, 16), (66000, 5, 70)]
 
 
@@ -108,7 +111,7 @@ def test_exact_products_on_each_tile_are_the_fused_reference(tk, orc, p, m, k, n
 
 @pytest.mark.parametrize("m,k,n,p", [((1 << 30) + 70, 1, 1, F32), ((1 << 26) + 70, 17, 3, F16)])
 def test_exact_products_of_more_rows_than_one_launch_takes(tk, orc, m, k, n, p):
-    """More than 2^32 threads' worth of rows (short sums), and more than one run of the ring's tiles: the
+    """More rows than 2^32 threads would take (short sums), which one launch cuts without an error, and more than one run of the ring's tiles: the
     fused reference's bits in rows around the runs' borders and the last ones, an accumulating output."""
     import torch
 
@@ -135,6 +138,52 @@ def test_exact_products_of_more_rows_than_one_launch_takes(tk, orc, m, k, n, p):
         rows = a[r0:r1].cpu().numpy().reshape(-1)
         assert orc.matmul(True, rows, k, r1 - r0, values, scales, p, n, k, want, n, None, NONE, 0.5, True) == 0
         assert np.array_equal(c[r0:r1].cpu().numpy().reshape(-1).view(np.uint32), want.view(np.uint32)), at
+
+
+@pytest.mark.parametrize("m,n", [(20, 40), (990, 1020)])  # one row block per workgroup and four
+@pytest.mark.parametrize("k", [12, 45, 864])  # short sums, a ragged stage, rounds of the ring and half a stage
+@pytest.mark.parametrize("p", [F32, F16, BF16, INT8, Q8_0])
+def test_exact_weights_that_widen_to_subnormals(tk, orc, p, k, m, n):
+    """Subnormal half and bfloat16 weights, quantised ones whose product with the scale is subnormal or
+    underflows, against inputs over the whole range of exponents, zeros of both signs, infinities and NaN:
+    the fused reference's bits (any NaN for a NaN)."""
+    import telmo_amd
+
+    from helpers import pack_q8_0
+
+    if p == Q8_0:
+        k = -(-k // 32) * 32
+    rng = np.random.default_rng(k + p)
+    a = np.ldexp(rng.uniform(-1, 1, (m, k)), rng.integers(-149, 60, (m, k))).astype(np.float32)
+    a[0], a[1], a[2] = -1e-30, 0.0, -0.0
+    a[3, k // 2], a[4, k - 1], a[5, 0] = np.inf, -np.inf, np.nan
+    # Rows whose sums stay subnormal.
+    low = (-149, -135) if p == F16 else (-25, -15)
+    a[6:13] = np.ldexp(rng.uniform(-1, 1, (7, k)), rng.integers(*low, (7, k))).astype(np.float32)
+    if p in (INT8, Q8_0):
+        q = rng.integers(-127, 128, (n, k)).astype(np.int8)
+        tiny = np.ldexp(1.0, rng.integers(-149, -120, (n, k // 32) if p == Q8_0 else n)).astype(np.float32)
+        values, scales = pack_q8_0(q, tiny) if p == Q8_0 else pack_int8(q, tiny)
+    else:  # F16's subnormals lie below 2^-14, the others' below 2^-126
+        low = -24 if p == F16 else -149
+        b = np.ldexp(rng.uniform(-1, 1, (n, k)), rng.integers(low, low + 30, (n, k))).astype(np.float32)
+        values, scales = orc.encode(b.reshape(-1), n, k, p)
+    want, got = np.zeros(m * n, np.float32), np.zeros(m * n, np.float32)
+    assert orc.matmul(True, a.reshape(-1), k, m, values, scales, p, n, k, want, n, None, NONE, 1.0, False) == 0
+    w = telmo_amd.PackedWeights.from_parts(tk, n, k, telmo_amd.Precision(p), values,
+                                           scales if scales is not None and len(scales) else None)
+    say("exact subnormal weights", p, m, k, n)
+    tk.set_mode(tk.EXACT)
+    try:
+        tk.linear(a.reshape(-1), m, w, got)
+    finally:
+        tk.set_mode(tk.FAST)
+        w.close()
+    nan = np.isnan(want)
+    assert np.array_equal(np.isnan(got), nan)
+    assert np.array_equal(got.view(np.uint32)[~nan], want.view(np.uint32)[~nan])
+    small = (np.abs(want) < np.finfo(np.float32).tiny) & (want != 0)
+    assert small.reshape(m, n)[6:13].any(axis=1).all()
 
 
 @pytest.mark.parametrize("k", [5, 16, 31, 64, 65, 200])
@@ -753,6 +802,41 @@ def test_rowmajor_right_hand_side_is_the_fused_reference(tk, orc, m, k, n, ldb):
         assert np.array_equal(cd.cpu().numpy().view(np.uint32), want.view(np.uint32)), (m, k, n, act)
     with pytest.raises(telmo_amd.TelmoError):  # one float short of the last panel
         tk.matmul_rowmajor_device(torch.from_numpy(a).cuda(), k, m, torch.from_numpy(b[:-1]).cuda(), k, n, ldb, cd, n)
+
+
+# Row blocks per workgroup 1 to 4, each with whole rounds of the ring and a ragged tail.
+@pytest.mark.parametrize("m,k,n", [(93, 769, 70), (375, 577, 1021), (750, 577, 1010), (1000, 577, 1021)])
+def test_rowmajor_tiles_are_the_fused_reference_at_any_alignment(tk, orc, m, k, n):
+    """Every tile on a view: rows of a, of the view and of c that are 16 bytes aligned, and each of them not
+    (odd strides, a base one float on, c with gaps that stay as they are)."""
+    import torch
+
+    import telmo_amd
+
+    rng = np.random.default_rng(m + k)
+    a, bias, npad = normal(rng, (m, k)), normal(rng, n), -(-n // 16) * 16
+    dense = normal(rng, (k, n))
+    values, _ = orc.encode(np.ascontiguousarray(dense.T), n, k, F32)
+    c0 = normal(rng, (m, n))
+    want = c0.copy()
+    assert orc.matmul(True, a.reshape(-1), k, m, values, None, F32, n, k, want.reshape(-1), n, bias, SILU, 0.5, True) == 0
+    epi = telmo_amd.Epilogue(bias=torch.from_numpy(bias).cuda(), act=telmo_amd.Act.SILU, scale=0.5, accumulate=True)
+
+    def view(x, ld, off):  # x's rows ld apart, off floats into a buffer of 7s
+        buf = torch.full((off + x.shape[0] * ld,), 7.0, device="cuda")
+        buf[off:].view(x.shape[0], ld)[:, :x.shape[1]] = torch.from_numpy(x).cuda()
+        return buf[off:]
+
+    up4 = lambda v: -(-v // 4) * 4  # noqa: E731
+    for odd_a, odd_b, odd_c in ((0, 0, 0), (1, 0, 0), (0, 1, 0), (0, 0, 1), (1, 1, 1)):
+        lda, ldb, ldc = up4(k) + odd_a, npad + 16 + odd_b, up4(n) + 4 + odd_c
+        ad, bd, cd = view(a, lda, odd_a), view(dense, ldb, odd_b), view(c0, ldc, odd_c)
+        say("rowmajor tile", m, k, n, odd_a, odd_b, odd_c)
+        tk.matmul_rowmajor_device(ad, lda, m, bd, k, n, ldb, cd, ldc, epi)
+        tk.synchronize()
+        got = cd.cpu().numpy().reshape(m, ldc)
+        assert np.array_equal(got[:, :n].view(np.uint32), want.view(np.uint32)), (odd_a, odd_b, odd_c)
+        assert np.all(got[:, n:] == 7.0), (odd_a, odd_b, odd_c)
 
 
 @pytest.mark.parametrize("m,k,n", [(750, 1024, 4096), (16, 640, 8198)])
