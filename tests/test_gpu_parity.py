@@ -111,8 +111,9 @@ def test_exact_products_on_each_tile_are_the_fused_reference(tk, orc, p, m, k, n
 
 @pytest.mark.parametrize("m,k,n,p", [((1 << 30) + 70, 1, 1, F32), ((1 << 26) + 70, 17, 3, F16)])
 def test_exact_products_of_more_rows_than_one_launch_takes(tk, orc, m, k, n, p):
-    """More rows than 2^32 threads would take (short sums), which one launch cuts without an error, and more than one run of the ring's tiles: the
-    fused reference's bits in rows around the runs' borders and the last ones, an accumulating output."""
+    """More rows than 2^32 threads would take (short sums), which one launch cuts without an error, and more
+    than one run of the ring's tiles: the fused reference's bits in rows around the runs' borders and the
+    last ones, an accumulating output."""
     import torch
 
     import telmo_amd
