@@ -34,8 +34,8 @@ struct RowsIn {
 // An output sink (class Out) takes the products after the epilogue. ROWS4 false: store(row, column, value),
 // for the rows there are. ROWS4 true, for sinks that need a lane's four rows together: begin(first row,
 // column, m) before a panel's products, so that what it reads then arrives under them, and store4(first
-// row, column, values, m) after, in every lane with a column; rows past m are the sink's to leave out
-// (with one row, only values[0] is computed).
+// row, column, values, m, one) after, in every lane with a column; rows past m are the sink's to leave out
+// (`one`, one row: only values[0] is computed).
 
 // Outputs stored to c (row stride ldc).
 struct StoreC {
@@ -391,12 +391,14 @@ __device__ __forceinline__ void mfma_body_impl(const In &in, Out &out, int m, in
                 fetch_panel<KBC>(wr, sc, bv, old, p + step, lane, wv, panel_stride, blk_stride, KB, scales, bias, c,
                                  ldc, N, m, accumulate, kw, KS);
         }
-        const int col = p * PANEL + ocol, rows = DOTR == 1 ? 1 : m;  // uniform
+        const int col = p * PANEL + ocol;
+        // One row: the k-split's is the dot4 body's, so its branch there is decided here.
+        const bool one = DOTR == 1 || (KS == 1 && m == 1);
         if (col < N && kw == 0) {
             float y[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
             for (int v = 0; v < 4; v++) {
-                if (Out::ROWS4 ? v == 0 || rows > 1 : orow + v < m) {
+                if (Out::ROWS4 ? v == 0 || !one : orow + v < m) {
                     float s;
                     if constexpr (Q8)
                         s = erow[v] == EXP_NONFINITE ? __builtin_nanf("") : __builtin_ldexpf(accq[v], -erow[v]);
@@ -406,7 +408,7 @@ __device__ __forceinline__ void mfma_body_impl(const In &in, Out &out, int m, in
                     if constexpr (!Out::ROWS4) out.store(orow + v, col, y[v]);
                 }
             }
-            if constexpr (Out::ROWS4) out.store4(orow, col, y, rows);
+            if constexpr (Out::ROWS4) out.store4(orow, col, y, m, one);
         }
     }
 }

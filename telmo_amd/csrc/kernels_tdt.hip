@@ -148,12 +148,12 @@ struct LstmOut {
         const int row = orow + (col & 3);
         c_old = s_in[at(row < m ? row : 0, col) + h];
     }
-    __device__ __forceinline__ void store4(int orow, int col, const float (&v)[4], int m) {
+    __device__ __forceinline__ void store4(int orow, int col, const float (&v)[4], int m, bool one) {
         const int k = col & 3, row = orow + k;
         float gate[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int r = 0; r < 4; r++) {
-            if (r > 0 && m == 1) break;
+            if (r > 0 && one) break;
             const float g[4] = {quad_lane<0>(v[r]), quad_lane<1>(v[r]), quad_lane<2>(v[r]), quad_lane<3>(v[r])};
 #pragma unroll
             for (int q = 0; q < 4; q++) gate[q] = k == r ? g[q] : gate[q];
