@@ -1023,9 +1023,9 @@ __global__ __launch_bounds__(RES_THREADS) void tdt_resident_kernel(ResArgs a) {
             // Wavefront w scores panels w, w + 4, ... of this workgroup, the weights as the first operand:
             // element v of lane l is row l % 16, column 4 (l / 16) + v, so a row's best entries meet over
             // a lane's four columns and then four lanes (with the rows first, over sixteen lanes for
-            // each of a lane's four rows: 60 s decoded 6960 us, so 6636). Each row keeps its best vocabulary entry and its best
-            // duration entry (index d for column vocab + d). A NaN first logit (column 0) is never
-            // beaten in the reference's argmax: it enters as (+inf, 0), which nothing comes before;
+            // each of a lane's four rows: 60 s decoded 6960 us, so 6636). Each row keeps its best
+            // vocabulary entry and its best duration entry (index d for column vocab + d). A NaN first
+            // logit (column 0) is never beaten in the reference's argmax: it enters as (+inf, 0), which nothing comes before;
             // a NaN first duration logit likewise.
             Key mine{0u, 0xffffffffu}, dmine{0u, 0xffffffffu};
             const int c4 = (lane >> 4) * 4, j16 = lane & 15;
@@ -1407,9 +1407,10 @@ __global__ void tdt_resident_init_kernel(uint64_t *words, int h, int layers, con
 // same tagged words between workgroups. The streams move in lockstep, one step for all: the joint
 // scores the TDT_ROWS row slots, TDT_ROWS / M (the stream's "slots") for each stream's window; the
 // decider walks each stream's window on its own and publishes one decision per stream; the streams
-// that emitted a token then run the prediction network together, as rows of an MFMA product (row j
-// is the j-th emitting stream), so a step costs about what one stream's step costs. Each stream's
-// words carry its own prediction count as tag, the step's words the step. int8 matrices.
+// that emitted a token then run the prediction network together, as rows of an MFMA product: stream q is
+// row q, the rows of the others are computed from whatever digits are there and not stored. Wavefront w
+// owns streams w and w + 4: it waits for their words and keeps their LSTM outputs in registers. Each
+// stream's words carry its own prediction count as tag, the step's words the step. int8 matrices.
 constexpr int MS_MAX = (int)TDT_MAX_STREAMS;
 
 struct MultiArgs {
