@@ -169,8 +169,7 @@ struct ExactArgs {
 // The epilogue and stores of RB blocks of 16 rows from m0 on and one panel: lane (lg, lj) holds columns
 // 4 lg + 0..3 of row lj of each block.
 template <int RB>
-__device__ __forceinline__ void store_blocks(const ExactArgs &g, const v4f (&acc)[RB], int m0, int panel) {
-    const int lane = threadIdx.x & 63, lg = lane >> 4, lj = lane & 15;
+__device__ __forceinline__ void store_blocks(const ExactArgs &g, const v4f (&acc)[RB], int m0, int panel, int lg, int lj) {
     const bool has_bias = g.epi.bias != nullptr, accumulate = g.epi.accumulate != 0;
     const int col = panel * PANEL + 4 * lg;
     if (col >= g.N) return;
@@ -439,7 +438,7 @@ __global__ __launch_bounds__(EXACT_THREADS) void exact_kernel(ExactArgs g) {
         else mma_ragged(f1, left - 32);
     }
 
-    store_blocks<RB>(g, acc, m0, panel);
+    store_blocks<RB>(g, acc, m0, panel, lg, lj);
 }
 
 // Sums of few inputs, without the ring: a wavefront takes 16 RB rows of one panel and loads its operands
@@ -485,7 +484,7 @@ __global__ __launch_bounds__(EXACT_THREADS) void exact_short_kernel(ExactArgs g)
             for (int r = 0; r < RB; r++) acc[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[s], a[r][s], acc[r], 0, 0, 0);
         }
     }
-    store_blocks<RB>(g, acc, m0, panel);
+    store_blocks<RB>(g, acc, m0, panel, lg, lj);
 }
 
 // launch(g) for runs of rows, whole blocks of `rows` of them: about RUN_GROUPS workgroups each, since HIP
